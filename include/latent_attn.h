@@ -226,7 +226,7 @@ int la_mla_decode(const la_decode_args* args, void* stream);
  * that size or schedule around the step and for tests. */
 enum {
   LA_PLAN_ATTENTION_VALU = 1, /* decode_generic_kernel (any dtype and head shape) */
-  LA_PLAN_ATTENTION_MFMA = 2  /* decode_mfma_kernel (kv_lora_rank 512, rope 64, 16-bit or FP8 cache, gfx950) */
+  LA_PLAN_ATTENTION_MFMA = 2  /* decode_mfma_kernel, or with few heads or rows decode_mfma16_kernel (kv_lora_rank 512, rope 64, 16-bit or FP8 cache, gfx950) */
 };
 enum {
   LA_PLAN_MERGE_VALU = 1,        /* combine_project_kernel */
@@ -244,7 +244,8 @@ typedef struct la_plan_info {
   int32_t chunk_rows;  /* rows per split-KV chunk */
   int32_t num_chunks;
   int32_t num_slots;   /* partial slots per query head: num_chunks + num_seqs - 1 */
-  int32_t head_groups; /* query-head groups per chunk (workgroups = num_chunks x head_groups, rounded for the XCDs) */
+  int32_t head_groups; /* groups of 128 query heads per chunk (one workgroup each, or eight where the plan's
+                          16-head MFMA kernel runs; the launch is rounded for the XCDs) */
   int32_t merge;       /* LA_PLAN_MERGE_* */
   int32_t absorb;      /* LA_PLAN_ABSORB_* */
   size_t workspace_bytes; /* la_mla_decode_workspace_size(args) */
@@ -264,8 +265,8 @@ int la_mla_decode_profiled(const la_decode_args* args, void* stream, void* event
 
 /* Streaming-ceiling measurement of the attention kernel's copy schedule. No
  * counterpart in the reference; for benchmarks and profilers. Runs, with the
- * plan la_mla_decode would use for `args`, a copies-only variant of the MFMA
- * attention kernel: the same grid and block mapping and, per 32-position
+ * plan la_mla_decode would use for `args`, a copies-only variant of the
+ * 128-head MFMA attention kernel: the same grid and block mapping and, per 32-position
  * tile, the same HBM->LDS copies of every wave (cache rows, k_rope rows,
  * RoPE table rows) into a ring of `ring` tile buffers (3: the kernel's own
  * ring; 4: the deepest one 160 KB of LDS holds), with one barrier per tile

@@ -54,6 +54,7 @@ enum Variant { kAuto = 0, kGeneric = 1, kMfma = 2 };
 
 struct Plan {
   bool mfma = false;
+  int waves16 = 0;  // 4 / 8: decode_mfma16_kernel with that many waves; 0: decode_mfma_kernel
   int chunk_len = 0;
   int num_chunks = 0;
   int num_slots = 0;
@@ -146,9 +147,22 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
 
   const int64_t total = paged ? p->total_rows : a->seq_offsets ? a->total_rows : (int64_t)a->num_seqs * a->seq_len;
   const int ncu = cu_count();
+  // Up to 32 query heads always take the 16-head kernel: 128-head workgroups
+  // run the matrix work of 128 heads whatever their number (32 x 4099 rows,
+  // attention us, 128-head against 16-head workgroups: 16 heads 51 / 33, 32
+  // heads 52 / 38, 64 heads 53 / 60).
+  const int heads16 = pl.mfma ? p->Hq / 16 : 0;
+  const bool few_heads = pl.mfma && heads16 <= 2;
   int64_t L;
   if (chunk_rows > 0) {
     L = chunk_rows;
+  } else if (few_heads) {
+    // two workgroups per CU and no more (16 heads x 131168 rows: 33.4 us with
+    // 257-row chunks, 37 with 128, 35.6 with 513); whole tiles only where a
+    // paged cache needs them, so that rounding leaves no CU without a chunk
+    const int64_t chunks = std::max<int64_t>(1, 2LL * ncu / heads16);
+    L = (total + chunks - 1) / chunks;
+    L = std::max<int64_t>((L + 15) / 16 * 16, 64);
   } else {
     int64_t groups = pl.mfma ? (p->Hq + mfma_heads_per_group() - 1) / mfma_heads_per_group() : p->Hq;
     int64_t target_blocks = pl.mfma ? ncu : 4LL * ncu;
@@ -178,6 +192,13 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
   if (nchunks > (int64_t)1 << 30) return LA_ERROR_INVALID_VALUE;
   pl.chunk_len = (int)L;
   pl.num_chunks = (int)nchunks;
+  // More heads take it while its workgroups fill the chip at most twice (the
+  // 128-head kernel would have a quarter of the CUs busy): 1 x 512 rows and
+  // 128 heads 16.2 us on the 128-head kernel, 7.9 here; 1 x 8192 17.0 / 11.6;
+  // four times that (16 queries over 2048 rows) 21.7 / 36.3. With at most one
+  // workgroup per CU, 8 waves take 128 positions per round trip.
+  if (pl.mfma && (few_heads || nchunks * heads16 <= 2 * ncu))
+    pl.waves16 = nchunks * heads16 <= ncu && L >= 128 ? 8 : 4;
   pl.num_slots = nchunks > 0 ? (int)(nchunks + a->num_seqs - 1) : 0;
 
   const int64_t tokens = (int64_t)a->num_seqs * a->queries_per_seq;
@@ -297,12 +318,16 @@ int run(const la_decode_args* a, hipStream_t stream, hipEvent_t ev_b = nullptr, 
     // the optional events bracket the attention kernel alone
     hipError_t e = hipSuccess;
     const int reps = repeat > 1 ? repeat : 1;
+    auto launch_mfma = [&](hipEvent_t b, hipEvent_t en) {
+      return plan.waves16 ? launch_decode_mfma16(p, plan.waves16, stream, b, en)
+                          : launch_decode_mfma(p, stream, b, en);
+    };
     if (plan.mfma && reps == 1) {
-      e = launch_decode_mfma(p, stream, ev_b, ev_e);  // recorded by the launch itself
+      e = launch_mfma(ev_b, ev_e);  // recorded by the launch itself
     } else {
       if (ev_b) e = hipEventRecord(ev_b, stream);
       for (int r = 0; r < reps && e == hipSuccess; ++r)
-        e = plan.mfma ? launch_decode_mfma(p, stream, nullptr, nullptr) : launch_decode_generic(p, stream);
+        e = plan.mfma ? launch_mfma(nullptr, nullptr) : launch_decode_generic(p, stream);
       if (e == hipSuccess && ev_e) e = hipEventRecord(ev_e, stream);
     }
     if (e != hipSuccess) return finish(e);

@@ -179,6 +179,43 @@ __device__ inline int find_seq(const DecodeProblem& p, int64_t r) {
   return lo;
 }
 
+// Block id -> (chunk, head group), XCD-aware. Workgroups are dispatched
+// round-robin over the 8 XCDs (id % 8), each with its own L2. The work items
+// (chunk, group), chunk-major, are cut into 8 contiguous ranges, one per XCD
+// (XCD x: items [x*per, (x+1)*per), id = 8 k + x is item x*per + k). With
+// one head group per chunk the chunks of one sequence share an L2, so the
+// sequence's Q rows are fetched from HBM once per XCD rather than once per
+// chunk, and every XCD streams one contiguous piece of the cache; with many
+// head groups (several queries over one cache) the groups of a chunk share an
+// L2 and its rows, and every XCD has work even when there are fewer chunks
+// than XCDs. Ids past the last item return at once (chunk >= num_chunks).
+__host__ __device__ inline int64_t mfma_grid_blocks(int num_chunks, int groups) {
+  return 8 * (((int64_t)num_chunks * groups + 7) / 8);
+}
+// 32-bit arithmetic: the grid (8 per blocks) is below 2^31, so every item
+// is (a 64-bit division here is ~130 dependent scalar instructions at the
+// kernel's start).
+__device__ inline void block_coords(int num_chunks, int groups, int* chunk, int* group) {
+  const uint32_t id = blockIdx.x;
+  const uint32_t per = ((uint32_t)num_chunks * (uint32_t)groups + 7) / 8;
+  const uint32_t item = (id & 7) * per + (id >> 3);
+  if (groups == 1) {
+    *group = 0;
+    *chunk = (int)item;
+  } else {
+    const uint32_t c = item / (uint32_t)groups;
+    *group = (int)(item - c * (uint32_t)groups);
+    *chunk = (int)c;
+  }
+}
+
+// find_seq for the MFMA kernels: with uniform sequences the row space is
+// below 2^31 rows (mfma_supported), so the division is a 32-bit one.
+__device__ inline int find_seq_mfma(const DecodeProblem& p, int64_t r) {
+  if (p.offsets) return find_seq(p, r);
+  return (int)((uint32_t)r / (uint32_t)p.seq_len);
+}
+
 // OCP FP8 E4M3 (e4m3fn) latent-cache element: sign, 4 exponent bits (bias
 // 7), 3 mantissa bits; exponent 0 is subnormal (m * 2^-9), 0x7F / 0xFF NaN.
 struct fp8e4m3 {
@@ -316,6 +353,10 @@ bool generic_supported(const DecodeProblem& p);
 hipError_t launch_decode_mfma(const DecodeProblem& p, hipStream_t stream, hipEvent_t ev_begin = nullptr,
                               hipEvent_t ev_end = nullptr);
 bool mfma_supported(const DecodeProblem& p);
+// The same with 16 query heads per workgroup (la_mfma16.hip); waves = 4 or 8
+// per workgroup (tiles of 64 or 128 positions).
+hipError_t launch_decode_mfma16(const DecodeProblem& p, int waves, hipStream_t stream, hipEvent_t ev_begin = nullptr,
+                                hipEvent_t ev_end = nullptr);
 // The attention kernel's grid and copy schedule with no compute (a
 // streaming-ceiling measurement); ring = 3 or 4 tile buffers. 16-bit
 // contiguous caches.
