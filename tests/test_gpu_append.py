@@ -190,3 +190,42 @@ def test_seq_lens_decode_equals_trimmed_cache(cuda, chunk_rows):
                             W_UK, W_UV, cos, sin, cfg)
     assert_close(out.cpu().numpy(), ref, "bf16", "seq_lens decode")
     assert_close(out2.cpu().numpy(), ref, "bf16", "packed decode")
+
+
+# around the launch's limit of one workgroup per sequence (4,096 groups of 8
+# elements: 56 tokens of 576), both sides, with a refused sequence, a base that
+# is not aligned for 8-element stores, and rotated queries
+@pytest.mark.parametrize("cache_dtype,src_dtype,bs,shift", [("bf16", "bf16", 0, 0), ("f16", "f32", 32, 0),
+                                                           ("f32", "bf16", 0, 1), ("bf16", "f32", 64, 0)])
+@pytest.mark.parametrize("tokens", [56, 57, 130])
+def test_append_prompt(cuda, cache_dtype, src_dtype, bs, shift, tokens):
+    cfg = MLAConfig.deepseek_v2()
+    B, cap, qps = 3, 192, 2
+    lens0 = [0, 61, 192 - tokens + 1]  # the last one has no room
+    g = torch.Generator().manual_seed(51)
+    flat = torch.randn(B * cap * ROW + 8, generator=g).to(TORCH_DTYPE[cache_dtype]).to(cuda)
+    kv = flat[shift:shift + B * cap * ROW].view(B * cap, ROW)
+    before = to_np(kv)
+    lens = torch.tensor(lens0, dtype=torch.int32, device=cuda)
+    status = torch.zeros(1, dtype=torch.int32, device=cuda)
+    c_t, k_rope = new_rows(B, tokens, src_dtype, 52)
+    q = torch.randn(B * qps, cfg.num_heads, 64, generator=g)
+    q_dev = q.to(cuda)
+    cos, sin = rope(cap, cfg, cuda)
+    kw = dict(q_rope=q_dev, rope_cos=cos, rope_sin=sin, status=status)
+    order = np.arange(B * cap)  # row of position p of sequence b: order[b * cap + p]
+    if bs:
+        table = torch.randperm(B * cap // bs, generator=g).to(torch.int32).view(B, -1)
+        order = (table.numpy().reshape(-1, 1) * bs + np.arange(bs)).reshape(-1)
+        F.append_kv(kv, lens, c_t.to(cuda), k_rope.to(cuda), cfg, block_table=table.to(cuda), block_size=bs, **kw)
+    else:
+        F.append_kv(kv.view(B, cap, ROW), lens, c_t.to(cuda), k_rope.to(cuda), cfg, **kw)
+    torch.cuda.synchronize()
+    want, want_lens, full = mo.append_rows(before[order], [0, cap, 2 * cap], [cap] * B, lens0, to_np(c_t), to_np(k_rope),
+                                           cache_dtype)
+    assert full and status.item() == 1 and lens.cpu().tolist() == list(want_lens)
+    assert np.array_equal(to_np(kv)[order], want)
+    rot = mo.rotate_queries(q.numpy().astype(np.float64), lens0, tokens, qps, to_np(cos), to_np(sin))
+    got = q_dev.cpu().numpy().astype(np.float64)
+    assert np.all(np.abs(got - rot)[:2 * qps] <= 1e-5 + 1e-5 * np.abs(rot)[:2 * qps])
+    assert torch.equal(q_dev[2 * qps:].cpu(), q[2 * qps:])
