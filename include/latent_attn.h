@@ -226,18 +226,21 @@ int la_mla_decode(const la_decode_args* args, void* stream);
  * that size or schedule around the step and for tests. */
 enum {
   LA_PLAN_ATTENTION_VALU = 1, /* decode_generic_kernel (any dtype and head shape) */
-  LA_PLAN_ATTENTION_MFMA = 2  /* decode_mfma_kernel, or with few heads or rows decode_mfma16_kernel (kv_lora_rank 512, rope 64, 16-bit or FP8 cache, gfx950) */
+  LA_PLAN_ATTENTION_MFMA = 2, /* decode_mfma_kernel, or with few heads or rows decode_mfma16_kernel (kv_lora_rank 512, rope 64, 16-bit or FP8 cache, gfx950) */
+  LA_PLAN_ATTENTION_MFMA_F32 = 3 /* decode_f32_kernel (float32 cache, the same dims) */
 };
 enum {
   LA_PLAN_MERGE_VALU = 1,        /* combine_project_kernel */
   LA_PLAN_MERGE_MFMA = 2,        /* merge_project_kernel: full partial rows per workgroup */
-  LA_PLAN_MERGE_MFMA_HALVES = 3  /* merge_project_half_kernel: latent halves added into the output */
+  LA_PLAN_MERGE_MFMA_HALVES = 3, /* merge_project_half_kernel: latent halves added into the output */
+  LA_PLAN_MERGE_MFMA_F32 = 4     /* merge_project_f32_kernel: float32 weights */
 };
 enum {
   LA_PLAN_ABSORB_NONE = 0,       /* queries come absorbed (q_absorbed) */
   LA_PLAN_ABSORB_VALU = 1,       /* absorb_kernel into fp32 q_abs */
   LA_PLAN_ABSORB_MFMA = 2,       /* absorb_mfma_kernel into fp32 q_abs */
-  LA_PLAN_ABSORB_MFMA_QPREP = 3  /* absorb_mfma_kernel straight into the attention kernel's 16-bit queries */
+  LA_PLAN_ABSORB_MFMA_QPREP = 3, /* absorb_mfma_kernel straight into the attention kernel's 16-bit queries */
+  LA_PLAN_ABSORB_MFMA_F32 = 4    /* absorb_f32_kernel: float32 weights */
 };
 typedef struct la_plan_info {
   int32_t attention;   /* LA_PLAN_ATTENTION_* (0 when num_seqs == 0) */

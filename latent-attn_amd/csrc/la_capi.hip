@@ -54,13 +54,16 @@ enum Variant { kAuto = 0, kGeneric = 1, kMfma = 2 };
 
 struct Plan {
   bool mfma = false;
+  bool f32 = false;  // decode_f32_kernel
   int waves16 = 0;  // 4 / 8: decode_mfma16_kernel with that many waves; 0: decode_mfma_kernel
   int chunk_len = 0;
   int num_chunks = 0;
   int num_slots = 0;
   bool proj_mfma = false;
+  bool proj_f32 = false;
   size_t part_scale_off = 0;
   bool absorb_mfma = false;  // q_nope . W_UK on the MFMA kernel
+  bool absorb_f32 = false;   // ... in fp32
   bool absorb_prep = false;  // ... writing the attention kernel's 16-bit Q rows directly
   size_t q_abs_off = 0, q_prep_off = 0, part_o_off = 0, part_lse_off = 0, total = 0;
 };
@@ -141,6 +144,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
   if (variant == kGeneric || !mfma_ok) {
     if (!generic_supported(*p)) return LA_ERROR_NOT_SUPPORTED;
     pl.mfma = false;
+    pl.f32 = variant == kAuto && decode_f32_supported(*p);
   } else {
     pl.mfma = true;
   }
@@ -156,6 +160,15 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
   int64_t L;
   if (chunk_rows > 0) {
     L = chunk_rows;
+  } else if (pl.f32) {
+    // two workgroups per CU, but no chunks under 128 rows while one per CU
+    // remains: their partial rows (2 KB per head) cost the merge more than the
+    // second workgroup gains (4 x 1000 rows, 128 heads: 51.5 us a step against
+    // 53.8 with 64; with 16 heads 43 against 36.5)
+    const int64_t groups = (p->Hq + 15) / 16;
+    const int64_t chunks = std::max<int64_t>(1, 2LL * ncu / groups);
+    L = std::max<int64_t>(((total + chunks - 1) / chunks + 15) / 16 * 16, 64);
+    if (L < 128 && groups * ((total + 127) / 128) >= ncu) L = 128;
   } else if (few_heads) {
     // two workgroups per CU and no more (16 heads x 131168 rows: 33.4 us with
     // 257-row chunks, 37 with 128, 35.6 with 513); whole tiles only where a
@@ -186,8 +199,8 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
     L = std::max<int64_t>(L, 64);
   }
   if (L > (int64_t)1 << 30) L = (int64_t)1 << 30;
-  if (pl.mfma && L > mfma_max_chunk_rows()) L = mfma_max_chunk_rows();
-  if (paged && pl.mfma) L = (L + 63) / 64 * 64;  // MFMA tiles start block-aligned
+  if ((pl.mfma || pl.f32) && L > mfma_max_chunk_rows()) L = mfma_max_chunk_rows();
+  if (paged && (pl.mfma || pl.f32)) L = (L + 63) / 64 * 64;  // MFMA tiles start block-aligned
   const int64_t nchunks = total > 0 ? (total + L - 1) / L : 0;
   if (nchunks > (int64_t)1 << 30) return LA_ERROR_INVALID_VALUE;
   pl.chunk_len = (int)L;
@@ -205,6 +218,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
   pl.absorb_mfma = absorb && absorb_mfma_supported(a->w_uk_dtype, c.num_heads, c.qk_nope_head_dim, c.kv_lora_rank) &&
                    (reinterpret_cast<uintptr_t>(a->q_nope) & 15) == 0 &&
                    (reinterpret_cast<uintptr_t>(a->W_UK) & 15) == 0;
+  pl.absorb_f32 = absorb && absorb_f32_supported(a->q_nope, a->W_UK, a->w_uk_dtype, c.qk_nope_head_dim, c.kv_lora_rank);
   pl.absorb_prep = pl.mfma && pl.absorb_mfma;
   size_t off = 0;
   if (absorb && !pl.absorb_prep) {
@@ -226,6 +240,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
   pl.part_lse_off = off;
   off += align_up((size_t)pl.num_slots * p->Hq * sizeof(float));
   pl.proj_mfma = project_mfma_supported(*p);
+  pl.proj_f32 = project_f32_supported(*p);
   pl.total = off;
 
   p->chunk_len = pl.chunk_len;
@@ -241,8 +256,9 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
 // 16-bit queries: the absorb kernel, or prep_q when the queries come
 // absorbed and there is at least one chunk).
 bool merge_halves(const DecodeProblem& p, const Plan& plan) {
-  return plan.proj_mfma && plan.mfma && (plan.absorb_prep || plan.num_chunks > 0) &&
-         merge_project_blocks(p) < cu_count();
+  const bool zeroed = plan.f32 ? plan.num_chunks > 0  // by decode_f32_kernel itself
+                               : plan.mfma && (plan.absorb_prep || plan.num_chunks > 0);
+  return zeroed && (plan.proj_f32 || (plan.proj_mfma && plan.mfma)) && merge_project_blocks(p) < cu_count();
 }
 
 // ev_b / ev_e (optional) are recorded around the attention kernel, which runs
@@ -297,7 +313,10 @@ int run(const la_decode_args* a, hipStream_t stream, hipEvent_t ev_b = nullptr, 
                              c.qk_nope_head_dim, c.kv_lora_rank, a->queries_per_seq, stream, zero_out, zero_n);
     } else {
       float* qa = reinterpret_cast<float*>(ws + plan.q_abs_off);
-      e = plan.absorb_mfma ? launch_absorb_mfma(a->q_nope, a->W_UK, a->w_uk_dtype, qa, 0, nullptr, 1.f, 0,
+      e = plan.absorb_f32 ? launch_absorb_f32(a->q_nope, a->W_UK, qa, (int)tokens, c.num_heads, c.qk_nope_head_dim,
+                                              c.kv_lora_rank, stream)
+          : plan.absorb_mfma
+              ? launch_absorb_mfma(a->q_nope, a->W_UK, a->w_uk_dtype, qa, 0, nullptr, 1.f, 0,
                                                 (int)tokens, c.num_heads, c.qk_nope_head_dim, c.kv_lora_rank, 1,
                                                 stream)
                            : launch_absorb(a->q_nope, a->W_UK, a->w_uk_dtype, qa, (int)tokens, c.num_heads,
@@ -327,12 +346,15 @@ int run(const la_decode_args* a, hipStream_t stream, hipEvent_t ev_b = nullptr, 
     } else {
       if (ev_b) e = hipEventRecord(ev_b, stream);
       for (int r = 0; r < reps && e == hipSuccess; ++r)
-        e = plan.mfma ? launch_mfma(nullptr, nullptr) : launch_decode_generic(p, stream);
+        e = plan.mfma ? launch_mfma(nullptr, nullptr)
+            : plan.f32 ? launch_decode_f32(p, stream, zero_out, zero_n)
+                       : launch_decode_generic(p, stream);
       if (e == hipSuccess && ev_e) e = hipEventRecord(ev_e, stream);
     }
     if (e != hipSuccess) return finish(e);
   }
-  return finish(plan.proj_mfma ? launch_combine_project_mfma(p, stream, merge_halves)
+  return finish(plan.proj_f32 ? launch_combine_project_f32(p, stream, merge_halves)
+                : plan.proj_mfma ? launch_combine_project_mfma(p, stream, merge_halves)
                                 : launch_combine_project(p, stream));
 }
 
@@ -432,15 +454,17 @@ int la_mla_decode_plan(const la_decode_args* args, la_plan_info* info) {
   *info = la_plan_info{};
   info->workspace_bytes = plan.total;
   if (args->num_seqs == 0) return LA_SUCCESS;
-  info->attention = plan.mfma ? LA_PLAN_ATTENTION_MFMA : LA_PLAN_ATTENTION_VALU;
+  info->attention = plan.mfma ? LA_PLAN_ATTENTION_MFMA : plan.f32 ? LA_PLAN_ATTENTION_MFMA_F32 : LA_PLAN_ATTENTION_VALU;
   info->chunk_rows = plan.chunk_len;
   info->num_chunks = plan.num_chunks;
   info->num_slots = plan.num_slots;
   info->head_groups = plan.mfma ? (p.Hq + la::mfma_heads_per_group() - 1) / la::mfma_heads_per_group() : p.Hq;
-  if (!plan.proj_mfma) info->merge = LA_PLAN_MERGE_VALU;
+  if (plan.proj_f32) info->merge = LA_PLAN_MERGE_MFMA_F32;
+  else if (!plan.proj_mfma) info->merge = LA_PLAN_MERGE_VALU;
   else info->merge = la::merge_halves(p, plan) ? LA_PLAN_MERGE_MFMA_HALVES : LA_PLAN_MERGE_MFMA;
   if (!args->q_nope) info->absorb = LA_PLAN_ABSORB_NONE;
   else if (plan.absorb_prep) info->absorb = LA_PLAN_ABSORB_MFMA_QPREP;
+  else if (plan.absorb_f32) info->absorb = LA_PLAN_ABSORB_MFMA_F32;
   else info->absorb = plan.absorb_mfma ? LA_PLAN_ABSORB_MFMA : LA_PLAN_ABSORB_VALU;
   return LA_SUCCESS;
 }
@@ -652,6 +676,11 @@ int la_absorb_q(const float* q_nope, const void* W_UK, int w_uk_dtype, float* q_
   if (!la::valid_cfg(cfg) || tokens < 0 || !la::valid_dtype(w_uk_dtype)) return LA_ERROR_INVALID_VALUE;
   if (tokens == 0) return LA_SUCCESS;
   if (!q_nope || !W_UK || !q_absorbed) return LA_ERROR_INVALID_VALUE;
+  if (la::absorb_f32_supported(q_nope, W_UK, w_uk_dtype, cfg->qk_nope_head_dim, cfg->kv_lora_rank)) {
+    const hipError_t f = la::launch_absorb_f32(q_nope, W_UK, q_absorbed, tokens, cfg->num_heads, cfg->qk_nope_head_dim,
+                                               cfg->kv_lora_rank, static_cast<hipStream_t>(stream));
+    return f == hipSuccess ? (int)LA_SUCCESS : la::record_hip(f);
+  }
   const bool mfma = la::absorb_mfma_supported(w_uk_dtype, cfg->num_heads, cfg->qk_nope_head_dim, cfg->kv_lora_rank) &&
                     (reinterpret_cast<uintptr_t>(q_nope) & 15) == 0 && (reinterpret_cast<uintptr_t>(W_UK) & 15) == 0;
   hipError_t e = mfma ? la::launch_absorb_mfma(q_nope, W_UK, w_uk_dtype, q_absorbed, 0, nullptr, 1.f, 0, tokens,

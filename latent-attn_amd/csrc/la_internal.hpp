@@ -347,6 +347,18 @@ hipError_t launch_append(const AppendProblem& p, hipStream_t stream);
 hipError_t launch_decode_generic(const DecodeProblem& p, hipStream_t stream);
 bool generic_supported(const DecodeProblem& p);
 
+// Whether the current device runs the MFMA kernels.
+bool device_is_gfx950();
+
+// fp32 split-KV decode and absorption on the fp32 MFMA (la_f32.hip): float32
+// caches with kv_lora_rank 512, qk_rope_head_dim 64; float32 weights. zero_out
+// (optional): zero_n floats the attention kernel zeroes for a half-row merge.
+bool decode_f32_supported(const DecodeProblem& p);
+hipError_t launch_decode_f32(const DecodeProblem& p, hipStream_t stream, float* zero_out = nullptr, int64_t zero_n = 0);
+bool absorb_f32_supported(const void* q_nope, const void* W_UK, int w_dtype, int dn, int dc);
+hipError_t launch_absorb_f32(const float* q_nope, const void* W_UK, float* q_abs, int tokens, int nh, int dn, int dc,
+                             hipStream_t stream);
+
 // MFMA split-KV decode for 16-bit and FP8 E4M3 caches with kv_lora_rank 512,
 // qk_rope_head_dim 64.
 // ev_begin / ev_end (optional) are recorded at the kernel's start and end.
@@ -389,6 +401,10 @@ int merge_project_blocks(const DecodeProblem& p);
 // which adds its product into p.out with atomics: p.out must be zero (fp16
 // partials only).
 hipError_t launch_combine_project_mfma(const DecodeProblem& p, hipStream_t stream, bool halves = false);
+
+// The same in fp32 for float32 weights; halves as above (any partial format).
+bool project_f32_supported(const DecodeProblem& p);
+hipError_t launch_combine_project_f32(const DecodeProblem& p, hipStream_t stream, bool halves);
 
 // q_abs = q_nope . W_UK per head.
 hipError_t launch_absorb(const float* q_nope, const void* W_UK, int w_dtype, float* q_abs, int tokens, int nh, int dn,

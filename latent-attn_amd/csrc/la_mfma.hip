@@ -1820,7 +1820,9 @@ hipError_t launch_t(const DecodeProblem& p, hipStream_t stream, hipEvent_t ev_be
   return hipGetLastError();
 }
 
-// The kernel uses gfx950-only instructions; cache the answer per device.
+}  // namespace
+
+// The MFMA kernels use gfx950-only instructions; the answer is cached per device.
 bool device_is_gfx950() {
   static std::mutex mu;
   static int cache[64] = {0};  // 0 unknown, 1 yes, 2 no
@@ -1834,8 +1836,6 @@ bool device_is_gfx950() {
   }
   return cache[dev] == 1;
 }
-
-}  // namespace
 
 int mfma_heads_per_group() { return kHG; }
 int mfma_max_chunk_rows() { return kMaxChunkRows; }

@@ -364,10 +364,11 @@ struct SlotRow<false> {
   }
 };
 
-// One fp16 slot's 4 columns of this lane (half-row merge).
+// One slot's 4 columns of this lane (half-row merge).
+template <bool F16>
 struct SlotRowHalf {
-  f16x4 h;
-  __device__ void load(const void* rowp) { h = *reinterpret_cast<const f16x4*>(rowp); }
+  typename std::conditional<F16, f16x4, f32x4>::type h;
+  __device__ void load(const void* rowp) { h = *reinterpret_cast<const decltype(h)*>(rowp); }
   __device__ void fma(float w, f32x4& o0, f32x4&) const {
 #pragma unroll
     for (int e = 0; e < 4; ++e) o0[e] += w * (float)h[e];
@@ -384,8 +385,8 @@ struct SlotRowHalf {
 // s = g, g + G, g + 2G, ... of row t, each weighted and divided by the sum
 // over ALL slots of the row, into this lane's 8 latent columns 8 lane ..
 // 8 lane + 7 (one wave per task), so the G tasks of a row sum to its merged O.
-// A half-row merge (fp16 slots) covers only the latent half c: 4 columns
-// 256 c + 4 lane .. +3 per lane, weighted with that half's row scale.
+// A half-row merge covers only the latent half c: 4 columns 256 c + 4 lane ..
+// +3 per lane, weighted (fp16 slots) with that half's row scale.
 // Rows past the batch and empty sequences give 0.
 struct MergeTask {
   int n = 0;       // slots of the row
@@ -419,9 +420,8 @@ __device__ inline MergeTask merge_task(const DecodeProblem& p, int t, int h, int
 template <bool F16, bool kHalf, int NB>
 __device__ inline void merge_tasks(const DecodeProblem& p, const int (&t)[2], int h, int g, int G, int lane,
                                    f32x4 (&o)[2][2], int c = 0) {
-  static_assert(F16 || !kHalf, "half-row merges read fp16 slots");
   typedef typename std::conditional<F16, _Float16, float>::type PT;
-  typedef typename std::conditional<kHalf, SlotRowHalf, SlotRow<F16>>::type SR;
+  typedef typename std::conditional<kHalf, SlotRowHalf<F16>, SlotRow<F16>>::type SR;
   const int64_t sstride = (int64_t)p.Hq * kDcP;
   static_assert(NB >= 1 && NB <= 64, "slot rows per batch");
   MergeTask mt[2];
@@ -751,6 +751,98 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_half_kernel(Decod
   LA_RSTAMP_WRITE(1);
 }
 
+// The same for float32 weights, all in fp32 (v_mfma_f32_16x16x4_f32): one
+// workgroup of 8 waves per (head h, 16 query rows), or, with kHalf and an
+// output zeroed earlier in the call, per latent half of it, the halves added
+// into the output as in merge_project_half_kernel. Half by half, the merged
+// rows go to LDS and meet W_UV's columns there; a step (jj, e) takes latent
+// column 16 jj + 4 (lane / 16) + e of the half, so both operands come in 16-B
+// loads. Bound by W_UV (33.5 MB at 128 heads) and the partial rows.
+// 4 tokens, 128 heads, 32 slots: 11.8 us; combine_project_kernel, which reduces
+// every output over a wave, 141.
+template <bool F16, bool kHalf>
+__global__ __launch_bounds__(kMPWaves * 64) void merge_project_f32_kernel(DecodeProblem p) {
+  constexpr int kNB = F16 || kHalf ? kMPSlots : kMPSlots / 2;  // fp32 rows, both halves: 8 in flight would spill
+  warm_kernarg_lines(p);
+  __shared__ __attribute__((aligned(16))) float orow[kMPRows * kMPHSum];  // merged half rows
+  __shared__ __attribute__((aligned(16))) float gp[kMPWaves * kMPHSum];   // slot-group sums
+  const int R = p.num_seqs * p.qps;
+  const int nrb = (R + kMPRows - 1) / kMPRows;
+  const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
+  const int k2 = kHalf ? k >> 1 : k;
+  const int h = (k2 / nrb) * 8 + x, rb = k2 % nrb;
+  if (h >= p.nh) return;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int rows = min(kMPRows, R - rb * kMPRows);
+  const float* const wrow = reinterpret_cast<const float*>(p.W_UV) +
+                            ((int64_t)h * p.dv + 16 * wave + (lane & 15)) * kDcP + 4 * (lane >> 4);
+  // sixteen accumulators, added as a tree: sums of 512 in one chain were further
+  // from 64 bits than the VALU kernel's
+  f32x4 part[16] = {};
+  const int c_first = kHalf ? (k & 1) : 0, c_end = kHalf ? c_first + 1 : 2;
+  for (int c = c_first; c < c_end; ++c) {
+    f32x4 bw[16];
+#pragma unroll
+    for (int jj = 0; jj < 16; ++jj) bw[jj] = *reinterpret_cast<const f32x4*>(wrow + 256 * c + 16 * jj);
+    if (c > c_first) __syncthreads();  // every wave is done with the first half's rows
+    f32x4 o[2][2];
+    if (rows >= kMPWaves) {
+      const int t[2] = {rb * kMPRows + wave, wave + kMPWaves < rows ? rb * kMPRows + wave + kMPWaves : -1};
+      merge_tasks<F16, true, kNB>(p, t, h, 0, 1, lane, o, c);
+      *reinterpret_cast<f32x4*>(&orow[wave * kMPHSum + 4 * lane]) = o[0][0];
+      *reinterpret_cast<f32x4*>(&orow[(wave + kMPWaves) * kMPHSum + 4 * lane]) =
+          t[1] >= 0 ? o[1][0] : f32x4{0.f, 0.f, 0.f, 0.f};
+    } else {
+      const int G = kMPWaves / rows;
+      const int r = wave / G, g = wave % G;
+      const int t[2] = {r < rows ? rb * kMPRows + r : -1, -1};
+      merge_tasks<F16, true, kNB>(p, t, h, g, G, lane, o, c);
+      *reinterpret_cast<f32x4*>(&gp[wave * kMPHSum + 4 * lane]) = o[0][0];
+      __syncthreads();
+      for (int i = tid; i < kMPRows * 64; i += kMPWaves * 64) {
+        const int rr = i / 64, c4 = i % 64;
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        if (rr < rows)
+          for (int q = 0; q < G; ++q) v += *reinterpret_cast<const f32x4*>(&gp[(rr * G + q) * kMPHSum + 4 * c4]);
+        *reinterpret_cast<f32x4*>(&orow[rr * kMPHSum + 4 * c4]) = v;
+      }
+    }
+    __syncthreads();
+    // A[m = lane % 16][latent column] from LDS, B[latent column][n = lane % 16] = W_UV
+#pragma unroll
+    for (int jj = 0; jj < 16; ++jj) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(&orow[(lane & 15) * kMPHSum + 16 * jj + 4 * (lane >> 4)]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f32x4& d = part[4 * (jj & 3) + e];
+        d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], bw[jj][e], d, 0, 0, 0);
+      }
+    }
+  }
+  // 16 wait states before the accumulators' first VALU reader: a branch may lie
+  // between the two, where the compiler adds none
+#pragma unroll
+  for (int i = 0; i < 16; i += 4)
+    asm volatile("s_nop 15" : "+v"(part[i]), "+v"(part[i + 1]), "+v"(part[i + 2]), "+v"(part[i + 3]));
+#pragma unroll
+  for (int n = 8; n > 0; n >>= 1)
+#pragma unroll
+    for (int i = 0; i < n; ++i) part[i] += part[i + n];
+  const f32x4 acc = part[0];
+  // D[m = 4 (lane / 16) + i][n = lane % 16]
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 4 * (lane >> 4) + i;
+    if (r < rows) {
+      const int t = rb * kMPRows + r;
+      const int64_t orow_i = (int64_t)(t / p.qps) * p.Hq + (t % p.qps) * p.nh + h;
+      float* const dst = &p.out[orow_i * p.dv + 16 * wave + (lane & 15)];
+      if constexpr (kHalf) atomicAdd(dst, acc[i]);
+      else *dst = acc[i];
+    }
+  }
+}
+
 }  // namespace
 
 bool absorb_mfma_supported(int w_dtype, int nh, int dn, int dc) {
@@ -782,6 +874,19 @@ hipError_t launch_absorb_mfma(const float* q_nope, const void* W_UK, int w_dtype
 bool project_mfma_supported(const DecodeProblem& p) {
   return (p.wuv_dtype == LA_DTYPE_BF16 || p.wuv_dtype == LA_DTYPE_F16) && p.dc == kDcP && p.dv == 128 &&
          (reinterpret_cast<uintptr_t>(p.W_UV) & 15) == 0;
+}
+
+bool project_f32_supported(const DecodeProblem& p) {
+  return p.wuv_dtype == LA_DTYPE_F32 && p.dc == kDcP && p.dv == 128 &&
+         (reinterpret_cast<uintptr_t>(p.W_UV) & 15) == 0 && device_is_gfx950();
+}
+
+hipError_t launch_combine_project_f32(const DecodeProblem& p, hipStream_t stream, bool halves) {
+  const dim3 grid((unsigned)((halves ? 2 : 1) * merge_project_blocks(p)));
+  auto k = p.part_f16 ? (halves ? merge_project_f32_kernel<true, true> : merge_project_f32_kernel<true, false>)
+                      : (halves ? merge_project_f32_kernel<false, true> : merge_project_f32_kernel<false, false>);
+  hipLaunchKernelGGL(k, grid, dim3(kMPWaves * 64), 0, stream, p);
+  return hipGetLastError();
 }
 
 int merge_project_blocks(const DecodeProblem& p) {

@@ -1,0 +1,85 @@
+"""The fp32 MFMA kernels (csrc/la_f32.hip, merge_project_f32_kernel) at their
+edges: tiles of 32 positions, 8 rows per wave, 16 heads per workgroup, 16
+query rows per merge, against the float64 oracle at the fp32 tolerance."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import assert_close
+from mla_cases import cfg_with_heads, make_queries, make_weights, rope, staircase_case, to_np
+from oracle import mla_oracle as mo
+
+pytestmark = pytest.mark.gpu
+
+
+def _dims(cfg):
+    return mo.Dims(cfg.d_model, 512, cfg.qk_nope_head_dim, 64, cfg.num_heads, 128)
+
+
+@pytest.mark.parametrize("layout", ["ragged", "paged"])
+@pytest.mark.parametrize("heads,chunk", [(1, 0), (16, 64), (20, 33), (32, 0)])
+def test_edges(cuda, layout, heads, chunk):
+    from latent_attn import functional as F
+
+    cfg = cfg_with_heads(heads)
+    lens = [1, 7, 8, 9, 31, 32, 33, 0, 63, 64, 65, 100, 5, 15, 16, 17, 40]  # 17 query rows: two merge blocks
+    B, bs, per = len(lens), 32, 4
+    W_UK, W_UV = make_weights(cfg, "f32", 3, cuda)
+    q_nope, q_rope = make_queries((B,), cfg, 4, cuda)
+    cos, sin = rope(max(lens), cfg, cuda)
+    g = torch.Generator().manual_seed(5)
+    seqs = [torch.randn(n, 576, generator=g) for n in lens]
+    if layout == "ragged":
+        off = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=cuda)
+        out = F.mla_decode(torch.cat(seqs).to(cuda), q_nope, q_rope, W_UK, W_UV, cos, sin, cfg, seq_offsets=off,
+                           chunk_rows=chunk)
+    else:
+        table = torch.randperm(B * per, generator=g).to(torch.int32).view(B, per)
+        pool = torch.full((B * per, bs, 576), 96.0)  # unfilled rows would show
+        for b, s in enumerate(seqs):
+            for p in range(0, len(s), bs):
+                pool[table[b, p // bs], :min(bs, len(s) - p)] = s[p:p + bs]
+        out = F.mla_decode(pool.view(-1, 576).to(cuda), q_nope, q_rope, W_UK, W_UV, cos, sin, cfg, chunk_rows=chunk,
+                           seq_lens=torch.tensor(lens, dtype=torch.int32, device=cuda), block_table=table.to(cuda),
+                           block_size=bs)
+    d = _dims(cfg)
+    off_np = np.concatenate([[0], np.cumsum(lens)]).tolist()
+    ref = mo.decode_sequences(to_np(torch.cat(seqs)), off_np, mo.absorb_q(to_np(q_nope), to_np(W_UK), d), to_np(q_rope),
+                              to_np(W_UV), to_np(cos), to_np(sin), d)
+    assert_close(out.cpu().numpy(), ref, "f32", f"f32 {layout} H={heads} chunk {chunk}")
+
+
+def test_rising_maximum_and_shared_cache(cuda):
+    """O rescaled as the maximum rises; absorbed queries; fp32 weights on both kinds of partial rows."""
+    from latent_attn import functional as F
+
+    cfg = cfg_with_heads(128)
+    kv, qa, qr = staircase_case(1, 300, "f32", 6, cuda)
+    _, W_UV = make_weights(cfg, "f32", 7, cuda)
+    cos, sin = rope(300, cfg, cuda)
+    d = _dims(cfg)
+    args = (to_np(qa), to_np(qr), to_np(W_UV), to_np(cos), to_np(sin), d)
+    out = F.fused_mla(kv[0], qa[0], qr[0], W_UV, cos, sin, cfg)
+    ref = mo.decode_sequences(to_np(kv[0]), [0, 300], *args)
+    assert_close(out.cpu().numpy()[None], ref, "f32", "f32 rising maximum")
+    kv16 = kv[0].to(torch.bfloat16)
+    out = F.fused_mla(kv16, qa[0], qr[0], W_UV, cos, sin, cfg)
+    ref = mo.decode_sequences(to_np(kv16), [0, 300], *args)
+    assert_close(out.cpu().numpy()[None], ref, "bf16", "bf16 cache, fp32 weights")
+
+
+@pytest.mark.parametrize("tokens,dn", [(1, 128), (16, 128), (17, 128), (3, 16), (5, 144)])
+def test_absorb(cuda, tokens, dn):
+    from latent_attn import functional as F
+
+    cfg = cfg_with_heads(3)
+    cfg.qk_nope_head_dim = dn
+    g = torch.Generator().manual_seed(8)
+    q = torch.randn(tokens, 3, dn, generator=g)
+    W = torch.randn(3 * dn, 512, generator=g)
+    got = F.absorb_q(q.to(cuda), W.to(cuda), cfg)
+    ref = np.einsum("thi,hic->thc", to_np(q), to_np(W).reshape(3, dn, 512))
+    assert_close(got.cpu().numpy(), ref, "f32", f"absorb f32 tokens {tokens} dn {dn}")
