@@ -354,7 +354,7 @@ int run(const la_decode_args* a, hipStream_t stream, hipEvent_t ev_b = nullptr, 
     if (e != hipSuccess) return finish(e);
   }
   return finish(plan.proj_f32 ? launch_combine_project_f32(p, stream, merge_halves)
-                : plan.proj_mfma ? launch_combine_project_mfma(p, stream, merge_halves)
+                : plan.proj_mfma ? launch_combine_project_mfma(p, stream, merge_halves, cu_count())
                                 : launch_combine_project(p, stream));
 }
 

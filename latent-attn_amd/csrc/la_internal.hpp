@@ -399,8 +399,8 @@ int merge_project_blocks(const DecodeProblem& p);
 // Merge of the split partials and W_UV projection in one kernel (the merged
 // rows stay in LDS: no workspace). halves: one workgroup per latent half,
 // which adds its product into p.out with atomics: p.out must be zero (fp16
-// partials only).
-hipError_t launch_combine_project_mfma(const DecodeProblem& p, hipStream_t stream, bool halves = false);
+// partials only). ncu: the device's compute units.
+hipError_t launch_combine_project_mfma(const DecodeProblem& p, hipStream_t stream, bool halves, int ncu);
 
 // The same in fp32 for float32 weights; halves as above (any partial format).
 bool project_f32_supported(const DecodeProblem& p);

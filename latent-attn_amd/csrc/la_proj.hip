@@ -408,7 +408,7 @@ __device__ inline MergeTask merge_task(const DecodeProblem& p, int t, int h, int
   return m;
 }
 
-// Merges up to two tasks (t[1] < 0: one) of the same slot group g of G.
+// Merges kTasks tasks (t[k] < 0: none) of the same slot group g of G.
 // Every load of both tasks goes out before anything waits: the first NB slot
 // rows of each task, each row's log-sum-exps (lane i: slot i, for the
 // maximum and the denominator) and the weights' inputs of the task's own
@@ -417,19 +417,19 @@ __device__ inline MergeTask merge_task(const DecodeProblem& p, int t, int h, int
 // groups of NB rows (and of 64 slots). Lane i's weights are broadcast with
 // v_readlane.
 // kHalf: half-row merge of latent half c (o[k][1] stays 0).
-template <bool F16, bool kHalf, int NB>
-__device__ inline void merge_tasks(const DecodeProblem& p, const int (&t)[2], int h, int g, int G, int lane,
-                                   f32x4 (&o)[2][2], int c = 0) {
+template <bool F16, bool kHalf, int NB, int kTasks>
+__device__ inline void merge_tasks(const DecodeProblem& p, const int (&t)[kTasks], int h, int g, int G, int lane,
+                                   f32x4 (&o)[kTasks][2], int c = 0) {
   typedef typename std::conditional<F16, _Float16, float>::type PT;
   typedef typename std::conditional<kHalf, SlotRowHalf<F16>, SlotRow<F16>>::type SR;
   const int64_t sstride = (int64_t)p.Hq * kDcP;
   static_assert(NB >= 1 && NB <= 64, "slot rows per batch");
-  MergeTask mt[2];
-  const PT* src[2];
-  SR d[2][NB];
-  float ls_all[2], ls_own[2], m_own[2], sa_own[2], sb_own[2];
+  MergeTask mt[kTasks];
+  const PT* src[kTasks];
+  SR d[kTasks][NB];
+  float ls_all[kTasks], ls_own[kTasks], m_own[kTasks], sa_own[kTasks], sb_own[kTasks];
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
+  for (int k = 0; k < kTasks; ++k) {
     mt[k] = merge_task(p, t[k], h, g, G);
     src[k] = reinterpret_cast<const PT*>(p.part_o) + mt[k].row0 * kDcP + (kHalf ? 256 * c + 4 * lane : 8 * lane);
 #pragma unroll
@@ -437,7 +437,7 @@ __device__ inline void merge_tasks(const DecodeProblem& p, const int (&t)[2], in
       if (u < mt[k].ns) d[k][u].load(src[k] + (int64_t)(g + G * u) * sstride);
   }
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
+  for (int k = 0; k < kTasks; ++k) {
     const float* lse = p.part_lse + mt[k].row0;
     ls_all[k] = lane < mt[k].n ? lse[(int64_t)lane * p.Hq] : -INFINITY;
     const bool own = lane < mt[k].ns;
@@ -450,7 +450,7 @@ __device__ inline void merge_tasks(const DecodeProblem& p, const int (&t)[2], in
     }
   }
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
+  for (int k = 0; k < kTasks; ++k) {
     o[k][0] = f32x4{0.f, 0.f, 0.f, 0.f};
     o[k][1] = o[k][0];
     const int n = mt[k].n, ns = mt[k].ns;
@@ -524,8 +524,9 @@ constexpr int kMPWaves = 8;
 // slot rows each task loads up front (one memory round trip for up to this
 // many; more loop over further batches, a round trip each). The half-row
 // merge also comes with 32 (8 B per lane each), launched when a task has
-// more than 8 slots (config 5: 32): more registers cost the short merges
-// (measured: configs 2 and 3 +1.5 us per step with 16 / 32 everywhere).
+// more than 16 slots (4 rows of 64 slots: 32 a task, 14.9 us against 19.5): its
+// 205 VGPRs leave one workgroup per CU, where 108 leave two (16 slots a task,
+// 16 rows: 18.4 us against 13.6).
 constexpr int kMPSlots = 8;
 constexpr int kMPPitch = kDcP + 4;  // floats per LDS row of a slot-group sum
 // 16-bit elements per LDS row of the high / low operand rows: 1040 B, 16 B
@@ -571,7 +572,7 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_kernel(DecodeProb
   f32x4 o[2][2];
   if (rows >= kMPWaves) {
     const int t[2] = {rb * kMPRows + wave, wave + kMPWaves < rows ? rb * kMPRows + wave + kMPWaves : -1};
-    merge_tasks<F16, false, kMPSlots>(p, t, h, 0, 1, lane, o);
+    merge_tasks<F16, false, kMPSlots, 2>(p, t, h, 0, 1, lane, o);
     LA_RSTAMP(2);
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
@@ -589,7 +590,7 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_kernel(DecodeProb
     const int G = kMPWaves / rows;
     const int r = wave / G, g = wave % G;
     const int t[2] = {r < rows ? rb * kMPRows + r : -1, -1};
-    merge_tasks<F16, false, kMPSlots>(p, t, h, g, G, lane, o);
+    merge_tasks<F16, false, kMPSlots, 2>(p, t, h, g, G, lane, o);
     LA_RSTAMP(2);
     *reinterpret_cast<f32x4*>(&gp[wave * kMPPitch + 8 * lane]) = o[0][0];
     *reinterpret_cast<f32x4*>(&gp[wave * kMPPitch + 8 * lane + 4]) = o[0][1];
@@ -642,7 +643,7 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_kernel(DecodeProb
 
 // Merge + W_UV projection over one latent half, for launches with fewer
 // (head, row block) workgroups than CUs (a few query rows): one workgroup of
-// 8 waves per (head h, 16 query rows, latent half c) merges the half rows
+// 8 waves per (head h, rpb <= 8 query rows, latent half c) merges the half rows
 // (fp16 slots, 512 B each) and multiplies them by W_UV's columns 256 c ..
 // 256 c + 255 (64 KB per head), so twice as many workgroups move half the
 // bytes each. Both halves add their products into out with float atomics;
@@ -654,7 +655,7 @@ constexpr int kMPHPitch = 256 + 8;  // 16-bit elements per LDS operand row (528 
 constexpr int kMPHSum = 256 + 4;    // floats per LDS row of a slot-group sum
 
 template <typename WT, int NB>
-__global__ __launch_bounds__(kMPWaves * 64) void merge_project_half_kernel(DecodeProblem p) {
+__global__ __launch_bounds__(kMPWaves * 64) void merge_project_half_kernel(DecodeProblem p, int rpb_log2) {
   LA_RSTAMP_DECL;
   LA_RSTAMP(0);
   warm_kernarg_lines(p);
@@ -667,7 +668,8 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_half_kernel(Decod
   __shared__ __attribute__((aligned(16))) short ol[kMPRows * kMPHPitch];  // and residuals
   __shared__ __attribute__((aligned(16))) float gp[kMPWaves * kMPHSum];   // slot-group sums
   const int R = p.num_seqs * p.qps;
-  const int nrb = (R + kMPRows - 1) / kMPRows;
+  const int rpb = 1 << rpb_log2;
+  const int nrb = (R + rpb - 1) >> rpb_log2;
   // id = 8 (2 (head / 8 * nrb + row block) + c) + head % 8: both halves of a
   // (head, row block) run on one XCD
   const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
@@ -675,7 +677,7 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_half_kernel(Decod
   const int h = (k2 / nrb) * 8 + x, rb = k2 % nrb;
   if (h >= p.nh) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int rows = min(kMPRows, R - rb * kMPRows);
+  const int rows = min(rpb, R - rb * rpb);
 
   // W_UV operands: B[k = 32 ks + 8 (lane / 16) + j][n = lane % 16]
   //              = W_UV[h dv + 16 wave + lane % 16][256 c + 32 ks + 8 (lane / 16) + j]
@@ -698,33 +700,25 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_half_kernel(Decod
     *reinterpret_cast<vec4*>(&oh[r * kMPHPitch + c0]) = hi;
     *reinterpret_cast<vec4*>(&ol[r * kMPHPitch + c0]) = lo;
   };
-  f32x4 o[2][2];
-  if (rows >= kMPWaves) {
-    const int t[2] = {rb * kMPRows + wave, wave + kMPWaves < rows ? rb * kMPRows + wave + kMPWaves : -1};
-    merge_tasks<true, true, NB>(p, t, h, 0, 1, lane, o, c);
-    LA_RSTAMP(2);
-    put4(wave, 4 * lane, o[0][0]);
-    put4(wave + kMPWaves, 4 * lane, t[1] >= 0 ? o[1][0] : f32x4{0.f, 0.f, 0.f, 0.f});
-    __syncthreads();
-  } else {
-    const int G = kMPWaves / rows;
-    const int r = wave / G, g = wave % G;
-    const int t[2] = {r < rows ? rb * kMPRows + r : -1, -1};
-    merge_tasks<true, true, NB>(p, t, h, g, G, lane, o, c);
-    LA_RSTAMP(2);
-    *reinterpret_cast<f32x4*>(&gp[wave * kMPHSum + 4 * lane]) = o[0][0];
-    __syncthreads();
-    // O half row r = sum of the G group rows of waves r G .. r G + G - 1; the
-    // block's other rows are zero
-    for (int i = tid; i < kMPRows * 64; i += kMPWaves * 64) {
-      const int rr = i / 64, c4 = i % 64;
-      f32x4 v = {0.f, 0.f, 0.f, 0.f};
-      if (rr < rows)
-        for (int q = 0; q < G; ++q) v += *reinterpret_cast<const f32x4*>(&gp[(rr * G + q) * kMPHSum + 4 * c4]);
-      put4(rr, 4 * c4, v);
-    }
-    __syncthreads();
+  // each row's slots over G = 8 / rows waves (rows <= 8)
+  const int G = kMPWaves / rows;
+  const int r = wave / G, g = wave % G;
+  const int t[1] = {r < rows ? rb * rpb + r : -1};
+  f32x4 o[1][2];
+  merge_tasks<true, true, NB, 1>(p, t, h, g, G, lane, o, c);
+  LA_RSTAMP(2);
+  *reinterpret_cast<f32x4*>(&gp[wave * kMPHSum + 4 * lane]) = o[0][0];
+  __syncthreads();
+  // O half row r = sum of the G group rows of waves r G .. r G + G - 1; the
+  // block's other rows are zero
+  for (int i = tid; i < kMPRows * 64; i += kMPWaves * 64) {
+    const int rr = i / 64, c4 = i % 64;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (rr < rows)
+      for (int q = 0; q < G; ++q) v += *reinterpret_cast<const f32x4*>(&gp[(rr * G + q) * kMPHSum + 4 * c4]);
+    put4(rr, 4 * c4, v);
   }
+  __syncthreads();
 
   // A[m = lane % 16][k = 32 ks + 8 (lane / 16) + j] = O[m][256 c + k] (high, low)
   LA_RSTAMP(3);
@@ -743,7 +737,7 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_half_kernel(Decod
   for (int i = 0; i < 4; ++i) {
     const int r = 4 * (lane >> 4) + i;
     if (r < rows) {
-      const int t = rb * kMPRows + r;
+      const int t = rb * rpb + r;
       const int64_t orow = (int64_t)(t / p.qps) * p.Hq + (t % p.qps) * p.nh + h;
       atomicAdd(&p.out[orow * p.dv + 16 * wave + (lane & 15)], acc_hi[i] + acc_lo[i] * (1.f / kLoScale));
     }
@@ -788,7 +782,7 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_f32_kernel(Decode
     f32x4 o[2][2];
     if (rows >= kMPWaves) {
       const int t[2] = {rb * kMPRows + wave, wave + kMPWaves < rows ? rb * kMPRows + wave + kMPWaves : -1};
-      merge_tasks<F16, true, kNB>(p, t, h, 0, 1, lane, o, c);
+      merge_tasks<F16, true, kNB, 2>(p, t, h, 0, 1, lane, o, c);
       *reinterpret_cast<f32x4*>(&orow[wave * kMPHSum + 4 * lane]) = o[0][0];
       *reinterpret_cast<f32x4*>(&orow[(wave + kMPWaves) * kMPHSum + 4 * lane]) =
           t[1] >= 0 ? o[1][0] : f32x4{0.f, 0.f, 0.f, 0.f};
@@ -796,7 +790,7 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_f32_kernel(Decode
       const int G = kMPWaves / rows;
       const int r = wave / G, g = wave % G;
       const int t[2] = {r < rows ? rb * kMPRows + r : -1, -1};
-      merge_tasks<F16, true, kNB>(p, t, h, g, G, lane, o, c);
+      merge_tasks<F16, true, kNB, 2>(p, t, h, g, G, lane, o, c);
       *reinterpret_cast<f32x4*>(&gp[wave * kMPHSum + 4 * lane]) = o[0][0];
       __syncthreads();
       for (int i = tid; i < kMPRows * 64; i += kMPWaves * 64) {
@@ -894,28 +888,35 @@ int merge_project_blocks(const DecodeProblem& p) {
   return 8 * ((p.nh + 7) / 8) * ((R + kMPRows - 1) / kMPRows);
 }
 
-hipError_t launch_combine_project_mfma(const DecodeProblem& p, hipStream_t stream, bool halves) {
+hipError_t launch_combine_project_mfma(const DecodeProblem& p, hipStream_t stream, bool halves, int ncu) {
   const int R = p.num_seqs * p.qps;
   if (R == 0) return hipSuccess;
   const int nrb = (R + kMPRows - 1) / kMPRows;
   if (halves) {
     if (!p.part_f16) return hipErrorInvalidValue;
     // id = 8 (2 (head / 8 * nrb + row block) + half) + head % 8
-    const dim3 grid((unsigned)(2 * merge_project_blocks(p)));
+    // Rows per workgroup: 8, one per wave (with 16, two: 16 rows x 16 slots x
+    // 128 heads took 16.0 us against 13.6), halved while the launch leaves CUs
+    // idle (32 rows x 17 slots x 16 heads: 9.9 us with 8 rows, 64 CUs; 7.5 with
+    // 4; 9.0 with 2, where workgroups pay their fixed part twice per CU).
+    const int hb = 2 * 8 * ((p.nh + 7) / 8);
+    int rpb_log2 = 3;
+    while (rpb_log2 > 0 && hb * ((R + (1 << rpb_log2) - 1) >> rpb_log2) < ncu) --rpb_log2;
+    const int rpb = 1 << rpb_log2;
+    const dim3 grid((unsigned)(hb * ((R + rpb - 1) >> rpb_log2)));
     // slots per task with equal sequences (seq_len / chunk_len when chunks
     // align with the sequences, else up to two more; rows of a block share
     // G = 8 / rows tasks); ragged or capacity caches keep the 8-slot batches
-    const int rows = R < kMPRows ? R : kMPRows;
-    const int G = rows >= kMPWaves ? 1 : kMPWaves / rows;
+    const int G = kMPWaves / (R < rpb ? R : rpb);
     const int64_t n = p.offsets || p.lens || p.chunk_len <= 0 ? 0
                       : p.seq_len % p.chunk_len == 0 ? p.seq_len / p.chunk_len
                                                      : p.seq_len / p.chunk_len + 2;
-    const bool wide = (n + G - 1) / G > kMPSlots;
+    const bool wide = (n + G - 1) / G > 2 * kMPSlots;
     auto k = p.wuv_dtype == LA_DTYPE_BF16 ? (wide ? merge_project_half_kernel<__hip_bfloat16, 32>
                                                   : merge_project_half_kernel<__hip_bfloat16, kMPSlots>)
                                           : (wide ? merge_project_half_kernel<__half, 32>
                                                   : merge_project_half_kernel<__half, kMPSlots>);
-    hipLaunchKernelGGL(k, grid, dim3(kMPWaves * 64), 0, stream, p);
+    hipLaunchKernelGGL(k, grid, dim3(kMPWaves * 64), 0, stream, p, rpb_log2);
     return hipGetLastError();
   }
   // id = 8 (head / 8 * nrb + row block) + head % 8
