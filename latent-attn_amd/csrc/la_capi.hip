@@ -330,7 +330,9 @@ int run(const la_decode_args* a, hipStream_t stream, hipEvent_t ev_b = nullptr, 
   p.part_scale = plan.mfma ? reinterpret_cast<float*>(ws + plan.part_scale_off) : nullptr;
   p.part_m = plan.mfma ? p.part_scale + (size_t)plan.num_slots * p.Hq * 2 : nullptr;
   if (plan.num_chunks > 0) {
-    if (plan.mfma && !plan.absorb_prep) {
+    if (plan.waves16 == 8 && !plan.absorb_prep) {
+      p.q_prep = nullptr;  // decode_mfma16_kernel takes the fp32 queries and zeroes the output
+    } else if (plan.mfma && !plan.absorb_prep) {
       hipError_t e = launch_prep_q(p, stream, zero_out, zero_n);
       if (e != hipSuccess) return finish(e);
     }
@@ -338,7 +340,7 @@ int run(const la_decode_args* a, hipStream_t stream, hipEvent_t ev_b = nullptr, 
     hipError_t e = hipSuccess;
     const int reps = repeat > 1 ? repeat : 1;
     auto launch_mfma = [&](hipEvent_t b, hipEvent_t en) {
-      return plan.waves16 ? launch_decode_mfma16(p, plan.waves16, stream, b, en)
+      return plan.waves16 ? launch_decode_mfma16(p, plan.waves16, stream, p.q_prep ? nullptr : zero_out, zero_n, b, en)
                           : launch_decode_mfma(p, stream, b, en);
     };
     if (plan.mfma && reps == 1) {

@@ -367,8 +367,10 @@ hipError_t launch_decode_mfma(const DecodeProblem& p, hipStream_t stream, hipEve
 bool mfma_supported(const DecodeProblem& p);
 // The same with 16 query heads per workgroup (la_mfma16.hip); waves = 4 or 8
 // per workgroup (tiles of 64 or 128 positions).
-hipError_t launch_decode_mfma16(const DecodeProblem& p, int waves, hipStream_t stream, hipEvent_t ev_begin = nullptr,
-                                hipEvent_t ev_end = nullptr);
+// With 8 waves and no q_prep it takes the fp32 queries; zero_out (optional): zero_n floats
+// it zeroes for a latent-half merge.
+hipError_t launch_decode_mfma16(const DecodeProblem& p, int waves, hipStream_t stream, float* zero_out, int64_t zero_n,
+                                hipEvent_t ev_begin = nullptr, hipEvent_t ev_end = nullptr);
 // The attention kernel's grid and copy schedule with no compute (a
 // streaming-ceiling measurement); ring = 3 or 4 tile buffers. 16-bit
 // contiguous caches.

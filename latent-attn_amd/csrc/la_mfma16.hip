@@ -50,6 +50,11 @@ constexpr int kDc = 512;
 constexpr int kDr = 64;
 constexpr int kRowElems = kDc + kDr;
 constexpr int kCtPitch = kDc * 2;       // 1024 B, chunks permuted by cf(row)
+// fp32 queries taken in (kW = 8): 8-element slots of a row, and its 16-bit LDS
+// pitch (73 16-B chunks: 16 rows at one chunk hit distinct banks)
+constexpr int kSlots = kRowElems / 8;
+constexpr int kQPitch = 2 * kRowElems + 16;
+
 // Workgroup of kW waves, tile of 16 kW positions, 16 query heads.
 template <int kW>
 struct Lds {
@@ -63,6 +68,7 @@ struct Lds {
   static constexpr int kStagePitch = 1040;
   static constexpr int kStat = 16 * kStagePitch;
   static_assert(kStat + 16 * 8 * kW <= kP, "epilogue staging fits the tile");
+  static_assert(kW != 8 || kRope + 16 * kQPitch <= kBytes, "the queries fit the k_rope and P rows");
   static_assert((8 / kW) * kBytes <= 160 * 1024, "two waves per SIMD");
 };
 
@@ -152,8 +158,17 @@ __device__ inline float sum_groups(float x) {
 }
 
 // KT: the MFMAs' type (bf16 for an FP8 cache). groups: workgroups per chunk.
+// kW = 8 takes absorbed queries as they come (p.q_prep == nullptr): the
+// workgroup scales and rounds its heads' rows as prep_q_kernel does and spreads
+// them over its waves through LDS, under the first tile's copies. One launch
+// less: 1 x 512 fp16 16.5 -> 14.8 us a call. (With every
+// wave reading the fp32 rows itself, 32 B of a row per lane, the call was 4.7 us
+// slower than with the launch.) kW = 4 has no room for it (its k_rope and P rows
+// are smaller than the queries). zero_out (optional): zero_n floats zeroed for
+// a half-row merge.
 template <typename KT, int kW, bool kPaged, bool kFp8>
-__global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem p, int groups) {
+__global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem p, int groups, float* zero_out,
+                                                                  int zero_n) {
   typedef Ops16<KT> O_;
   typedef typename O_::vec vec;
   typedef typename O_::elem E;
@@ -172,6 +187,8 @@ __global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
   lchar* L = (lchar*)lds_raw;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (zero_out)
+    for (int i = blockIdx.x * 64 * kW + threadIdx.x; i < zero_n; i += gridDim.x * 64 * kW) zero_out[i] = 0.f;
   int chunk, group;
   block_coords(p.num_chunks, groups, &chunk, &group);
   if (chunk >= p.num_chunks) return;
@@ -200,16 +217,32 @@ __global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem
     const int ntiles = last / kT + 1;
     const int rlim = p.rope_rows > 0 ? (int)(p.rope_rows - 1) : INT32_MAX;
 
-    // Q^T as the B operand: lane holds Q[head0 + n16][32kk + 8g .. +8]
-    // (q_prep in operand order, qprep_index)
+    // Q^T as the B operand: lane holds Q[head0 + n16][32kk + 8g .. +8], from
+    // q_prep (in operand order, qprep_index), or from the fp32 queries' slots
+    // (8 elements each) tid, tid + 512, tid + 1024, which go through LDS below
     vec q[18];
-    {
+    const bool q32 = kW == 8 && !p.q_prep;
+    f32x4 qf[kW == 8 ? 6 : 1];
+    if (!q32) {
       const int ql = fresh_lane();
       const int64_t qrow = (int64_t)s * qprep_rows_per_seq(p.Hq) + head0 + (ql & 15);
-      const vec* qs = reinterpret_cast<const vec*>(reinterpret_cast<const E*>(p.q_prep) + qprep_index(qrow, 0)) +
-                      64 * (ql >> 5) + 32 * ((ql >> 4) & 1);
+      const vec* qs =
+          reinterpret_cast<const vec*>(reinterpret_cast<const E*>(p.q_prep) + qprep_index(qrow, 8 * (ql >> 4)));
 #pragma unroll
       for (int kk = 0; kk < 18; ++kk) q[kk] = qs[128 * kk];
+    }
+    if constexpr (kW == 8) {
+      if (q32) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const int slot = min((int)threadIdx.x + 512 * i, 16 * kSlots - 1);
+          const int row = slot / kSlots, j = slot - row * kSlots;
+          const int64_t hq = (int64_t)s * p.Hq + head0 + row;
+          const float* src = j < kDc / 8 ? p.q_abs + hq * kDc + 8 * j : p.q_rope + hq * kDr + 8 * (j - kDc / 8);
+          qf[2 * i] = reinterpret_cast<const f32x4*>(src)[0];
+          qf[2 * i + 1] = reinterpret_cast<const f32x4*>(src)[1];
+        }
+      }
     }
     f32x4 o[kCB];
     float m = -INFINITY, l = 0.f;
@@ -260,6 +293,27 @@ __global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem
         for (int j = 0; j < 16; ++j)
           __builtin_amdgcn_global_load_lds(base + (uint32_t)(min(j, left) * kRowB + 16 * (ln ^ cf(j))),
                                            (lds_void*)(L + (16 * wave + j) * kCtPitch), 16, 0, 0);
+      }
+      if constexpr (kW == 8) {
+        if (q32 && t == 0) {  // the queries, in the place of the k_rope and P rows
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            const int slot = (int)threadIdx.x + 512 * i;
+            const int row = slot / kSlots, j = slot - row * kSlots;
+            vec v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              v[e] = (E)(qf[2 * i][e] * p.scale_log2);
+              v[4 + e] = (E)(qf[2 * i + 1][e] * p.scale_log2);
+            }
+            if (slot < 16 * kSlots) lds_st(L, D::kRope + row * kQPitch + 16 * j, v);
+          }
+          lds_barrier();
+#pragma unroll
+          for (int kk = 0; kk < 18; ++kk)
+            q[kk] = lds_ld<vec>(L, D::kRope + (ln & 15) * kQPitch + 64 * kk + 16 * (ln >> 4));
+          lds_barrier();
+        }
       }
       {
         i16x8 ra, rb;
@@ -442,7 +496,8 @@ __global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem
 }
 
 template <typename KT, int kW, bool kPaged, bool kFp8>
-hipError_t launch16_t(const DecodeProblem& p, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
+hipError_t launch16_t(const DecodeProblem& p, hipStream_t stream, float* zero_out, int zero_n, hipEvent_t ev_begin,
+                      hipEvent_t ev_end) {
   constexpr int lds = Lds<kW>::kBytes;
   static bool attr_set = false;  // per instance; setting it twice is harmless
   if (!attr_set) {
@@ -455,30 +510,34 @@ hipError_t launch16_t(const DecodeProblem& p, hipStream_t stream, hipEvent_t ev_
   const dim3 grid((unsigned)mfma_grid_blocks(p.num_chunks, groups));
   if (ev_begin || ev_end)
     hipExtLaunchKernelGGL((decode_mfma16_kernel<KT, kW, kPaged, kFp8>), grid, dim3(64 * kW), lds, stream, ev_begin,
-                          ev_end, 0, p, groups);
+                          ev_end, 0, p, groups, zero_out, zero_n);
   else
-    hipLaunchKernelGGL((decode_mfma16_kernel<KT, kW, kPaged, kFp8>), grid, dim3(64 * kW), lds, stream, p, groups);
+    hipLaunchKernelGGL((decode_mfma16_kernel<KT, kW, kPaged, kFp8>), grid, dim3(64 * kW), lds, stream, p, groups, zero_out,
+                       zero_n);
   return hipGetLastError();
 }
 
 template <int kW>
-hipError_t launch16_w(const DecodeProblem& p, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
+hipError_t launch16_w(const DecodeProblem& p, hipStream_t stream, float* zero_out, int zero_n, hipEvent_t ev_begin,
+                      hipEvent_t ev_end) {
   typedef __hip_bfloat16 B;
   if (p.block_table) {
-    if (p.kv_dtype == LA_DTYPE_FP8_E4M3) return launch16_t<B, kW, true, true>(p, stream, ev_begin, ev_end);
-    if (p.kv_dtype == LA_DTYPE_BF16) return launch16_t<B, kW, true, false>(p, stream, ev_begin, ev_end);
-    return launch16_t<__half, kW, true, false>(p, stream, ev_begin, ev_end);
+    if (p.kv_dtype == LA_DTYPE_FP8_E4M3) return launch16_t<B, kW, true, true>(p, stream, zero_out, zero_n, ev_begin, ev_end);
+    if (p.kv_dtype == LA_DTYPE_BF16) return launch16_t<B, kW, true, false>(p, stream, zero_out, zero_n, ev_begin, ev_end);
+    return launch16_t<__half, kW, true, false>(p, stream, zero_out, zero_n, ev_begin, ev_end);
   }
-  if (p.kv_dtype == LA_DTYPE_FP8_E4M3) return launch16_t<B, kW, false, true>(p, stream, ev_begin, ev_end);
-  if (p.kv_dtype == LA_DTYPE_BF16) return launch16_t<B, kW, false, false>(p, stream, ev_begin, ev_end);
-  return launch16_t<__half, kW, false, false>(p, stream, ev_begin, ev_end);
+  if (p.kv_dtype == LA_DTYPE_FP8_E4M3) return launch16_t<B, kW, false, true>(p, stream, zero_out, zero_n, ev_begin, ev_end);
+  if (p.kv_dtype == LA_DTYPE_BF16) return launch16_t<B, kW, false, false>(p, stream, zero_out, zero_n, ev_begin, ev_end);
+  return launch16_t<__half, kW, false, false>(p, stream, zero_out, zero_n, ev_begin, ev_end);
 }
 
 }  // namespace
 
-hipError_t launch_decode_mfma16(const DecodeProblem& p, int waves, hipStream_t stream, hipEvent_t ev_begin,
-                                hipEvent_t ev_end) {
-  return waves == 8 ? launch16_w<8>(p, stream, ev_begin, ev_end) : launch16_w<4>(p, stream, ev_begin, ev_end);
+hipError_t launch_decode_mfma16(const DecodeProblem& p, int waves, hipStream_t stream, float* zero_out, int64_t zero_n,
+                                hipEvent_t ev_begin, hipEvent_t ev_end) {
+  if (zero_n > INT32_MAX / 2) return hipErrorInvalidValue;  // the kernel counts in 32 bits
+  return waves == 8 ? launch16_w<8>(p, stream, zero_out, (int)zero_n, ev_begin, ev_end)
+                    : launch16_w<4>(p, stream, zero_out, (int)zero_n, ev_begin, ev_end);
 }
 
 }  // namespace la
