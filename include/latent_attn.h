@@ -139,8 +139,10 @@ typedef struct la_decode_args {
   /* optional DEVICE int32 array of num_seqs lengths (as la_append_kv keeps
    * them): sequence s is the first seq_lens[s] rows of its region above
    * (clamped into it; rows past it are unfilled capacity and are not read).
-   * NULL: each sequence is its whole region. The split plan covers the
-   * regions, so capacity far beyond the lengths costs idle blocks. */
+   * NULL: each sequence is its whole region. The MFMA kernels cut the
+   * filled rows (unless chunk_rows is given, or there are fewer than four
+   * chunks per sequence); otherwise the split plan covers the regions, so
+   * capacity far beyond the lengths costs idle blocks. */
   const int32_t* seq_lens;
   /* optional paged cache (block tables): kv_cache is then a pool of
    * total_rows rows in blocks of block_size rows (total_rows a multiple of
@@ -244,7 +246,7 @@ enum {
 };
 typedef struct la_plan_info {
   int32_t attention;   /* LA_PLAN_ATTENTION_* (0 when num_seqs == 0) */
-  int32_t chunk_rows;  /* rows per split-KV chunk */
+  int32_t chunk_rows;  /* rows per split-KV chunk (of the regions; shorter on the device with seq_lens) */
   int32_t num_chunks;
   int32_t num_slots;   /* partial slots per query head: num_chunks + num_seqs - 1 */
   int32_t head_groups; /* groups of 128 query heads per chunk (one workgroup each, or eight where the plan's

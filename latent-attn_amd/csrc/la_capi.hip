@@ -157,7 +157,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
   // heads 52 / 38, 64 heads 53 / 60).
   const int heads16 = pl.mfma ? p->Hq / 16 : 0;
   const bool few_heads = pl.mfma && heads16 <= 2;
-  int64_t L;
+  int64_t L, min_rows = 64;
   if (chunk_rows > 0) {
     L = chunk_rows;
   } else if (pl.f32) {
@@ -169,6 +169,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
     const int64_t chunks = std::max<int64_t>(1, 2LL * ncu / groups);
     L = std::max<int64_t>(((total + chunks - 1) / chunks + 15) / 16 * 16, 64);
     if (L < 128 && groups * ((total + 127) / 128) >= ncu) L = 128;
+    min_rows = std::min<int64_t>(L, 128);
   } else if (few_heads) {
     // two workgroups per CU and no more (16 heads x 131168 rows: 33.4 us with
     // 257-row chunks, 37 with 128, 35.6 with 513); whole tiles only where a
@@ -192,8 +193,10 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
     // one cache), each writing its own partials, so the floor is per group.
     if (pl.mfma) {
       const int64_t hg = std::min<int64_t>(p->Hq, mfma_heads_per_group());
-      L = std::max<int64_t>(L, (hg * c.kv_lora_rank + c.kv_lora_rank + c.qk_rope_head_dim - 1) /
-                                   (c.kv_lora_rank + c.qk_rope_head_dim));
+      const int64_t rows = (hg * c.kv_lora_rank + c.kv_lora_rank + c.qk_rope_head_dim - 1) /
+                           (c.kv_lora_rank + c.qk_rope_head_dim);
+      L = std::max<int64_t>(L, rows);
+      min_rows = std::max<int64_t>((rows + 63) / 64 * 64, 64);
     }
     L = (L + 63) / 64 * 64;
     L = std::max<int64_t>(L, 64);
@@ -238,12 +241,23 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
     off += align_up((size_t)pl.num_slots * p->Hq * 3 * sizeof(float));
   }
   pl.part_lse_off = off;
-  off += align_up((size_t)pl.num_slots * p->Hq * sizeof(float));
+  const bool filled = a->seq_lens && chunk_rows == 0 && (pl.mfma || pl.f32) && 4LL * a->num_seqs <= nchunks &&
+                      total <= INT32_MAX;
+  off += align_up((size_t)pl.num_slots * p->Hq * sizeof(float) +
+                  (filled ? ((size_t)a->num_seqs + 1) * sizeof(int32_t) : 0));  // filled_notes
   pl.proj_mfma = project_mfma_supported(*p);
   pl.proj_f32 = project_f32_supported(*p);
   pl.total = off;
 
   p->chunk_len = pl.chunk_len;
+  // Per-sequence lengths: the chunks are pieces of the sequences' filled rows
+  // (seq_in_plan), down to the plan's shortest chunk, while there are four or
+  // more per sequence (100 sequences of 100 to 4000 rows over 256 chunks, too
+  // uneven pieces: 165 us a step against 147 over their 4096-row regions; 64 of
+  // 300 to 8192: 120 against 154; 32 of 500 to 8000 in 32768-row regions: 74
+  // against 208).
+  if (filled)
+    p->chunk_len = -(int)std::min<int64_t>((min_rows + 31) / 32 * 32, L);
   p->num_chunks = pl.num_chunks;
   p->num_slots = pl.num_slots;
   *plan = pl;
@@ -489,6 +503,7 @@ int la_stream_ceiling(const la_decode_args* args, int32_t ring, void* stream, vo
   if (!plan.mfma || p.block_table || (p.kv_dtype != LA_DTYPE_BF16 && p.kv_dtype != LA_DTYPE_F16))
     return LA_ERROR_NOT_SUPPORTED;
   if (plan.num_chunks == 0) return LA_SUCCESS;
+  p.chunk_len = plan.chunk_len;  // the copies walk the regions
   const hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e = hipSuccess;
   if (event_begin) e = hipEventRecord(static_cast<hipEvent_t>(event_begin), s);

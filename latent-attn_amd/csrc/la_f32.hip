@@ -62,7 +62,7 @@ __device__ inline f32x4 mma(float a, float b, f32x4 c) { return __builtin_amdgcn
 // (the compiler adds none where a branch lies between the two).
 __device__ inline void settle(f32x4& d) { asm volatile("s_nop 15" : "+v"(d)); }
 
-template <bool kPaged>
+template <bool kPaged, bool kFilled>
 __global__ __launch_bounds__(kThreads, 2) void decode_f32_kernel(DecodeProblem p, int groups, float* zero_out,
                                                                  int64_t zero_n) {
   warm_kernarg_lines(p);
@@ -80,29 +80,17 @@ __global__ __launch_bounds__(kThreads, 2) void decode_f32_kernel(DecodeProblem p
   if (chunk >= p.num_chunks) return;
   const int head0 = group * 16;
 
-  const int64_t end_all = seq_begin(p, p.num_seqs);
-  int64_t lo = (int64_t)chunk * p.chunk_len;
-  const int64_t hi = min(lo + (int64_t)p.chunk_len, end_all);
-  lo = max(lo, seq_begin(p, 0));
-  if (lo >= hi) return;
-  int s = find_seq_mfma(p, lo);
+  ChunkWalk<kFilled> w;
+  if (!walk_begin(p, chunk, group, w)) return;
 
   const int pb_w = wave & 1, kh = wave >> 1;  // this wave's score block and half of the row
   const int row_l = 16 * pb_w + n16;
 
-  while (lo < hi) {
-    const int64_t s_lo = seq_begin(p, s);
-    lo = max(lo, s_lo);  // past the unfilled rows of the previous region
-    if (lo >= hi) break;
-    const int64_t s_hi = seq_end(p, s);
-    if (s_hi <= lo) {  // empty sequence, or lo in its unfilled rows
-      if (++s >= p.num_seqs) break;
-      continue;
-    }
-    const int64_t seg_hi = min(hi, s_hi);
-    const char* const seg_base = reinterpret_cast<const char*>(p.kv) + (kPaged ? 0 : lo * kRowB);
-    const uint32_t pos0 = (uint32_t)(lo - s_lo);
-    const int last = (int)(seg_hi - lo - 1);
+  while (walk_next(p, w)) {
+    const int s = w.s;
+    const char* const seg_base = reinterpret_cast<const char*>(p.kv) + (kPaged ? 0 : (w.row0 + (w.lo - w.s_lo)) * kRowB);
+    const uint32_t pos0 = (uint32_t)(w.lo - w.s_lo);
+    const int last = (int)(w.seg_hi - w.lo - 1);
     const int ntiles = last / kT + 1;
     const int64_t rlim = p.rope_rows > 0 ? p.rope_rows - 1 : INT64_MAX;
 
@@ -259,8 +247,8 @@ __global__ __launch_bounds__(kThreads, 2) void decode_f32_kernel(DecodeProblem p
       if (wave == 0 && g == 0) p.part_lse[row] = m + log2f(l);
     }
     lds_barrier();  // the next segment's tile lands on this one's
-    lo = seg_hi;
-    ++s;
+    w.lo = w.seg_hi;
+    ++w.s;
   }
 }
 
@@ -327,17 +315,17 @@ __global__ __launch_bounds__(256) void absorb_f32_kernel(const float* __restrict
     *reinterpret_cast<f32x4*>(dst + 4 * r) = f32x4{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
 }
 
-template <bool kPaged>
+template <bool kPaged, bool kFilled>
 hipError_t launch_f32_t(const DecodeProblem& p, hipStream_t stream, float* zero_out, int64_t zero_n) {
   static bool attr_set = false;  // per instance; setting it twice is harmless
   if (!attr_set) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_f32_kernel<kPaged>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_f32_kernel<kPaged, kFilled>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     if (e != hipSuccess) return e;
     attr_set = true;
   }
   const int groups = (p.Hq + 15) / 16;
-  hipLaunchKernelGGL(decode_f32_kernel<kPaged>, dim3((unsigned)mfma_grid_blocks(p.num_chunks, groups)), dim3(kThreads),
+  hipLaunchKernelGGL((decode_f32_kernel<kPaged, kFilled>), dim3((unsigned)mfma_grid_blocks(p.num_chunks, groups)), dim3(kThreads),
                      kLdsBytes, stream, p, groups, zero_out, zero_n);
   return hipGetLastError();
 }
@@ -354,8 +342,9 @@ bool decode_f32_supported(const DecodeProblem& p) {
 }
 
 hipError_t launch_decode_f32(const DecodeProblem& p, hipStream_t stream, float* zero_out, int64_t zero_n) {
-  return p.block_table ? launch_f32_t<true>(p, stream, zero_out, zero_n)
-                       : launch_f32_t<false>(p, stream, zero_out, zero_n);
+  if (p.block_table) return launch_f32_t<true, true>(p, stream, zero_out, zero_n);
+  return p.chunk_len < 0 ? launch_f32_t<false, true>(p, stream, zero_out, zero_n)
+                         : launch_f32_t<false, false>(p, stream, zero_out, zero_n);
 }
 
 bool absorb_f32_supported(const void* q_nope, const void* W, int w_dtype, int dn, int dc) {

@@ -172,18 +172,17 @@ __global__ __launch_bounds__(kCombineThreads) void combine_project_kernel(Decode
     float* orow = Os + rr * dc;
     const int r = r0 + rr;
     int64_t lo = 0, hi = 0;
-    int s = 0, hq = 0;
+    int s = 0, hq = 0, len = 1;
     if (r < R) {
       s = r / p.qps;
       hq = (r % p.qps) * p.nh + h;
-      lo = seq_begin(p, s);
-      hi = seq_end(p, s);
+      len = seq_in_plan(p, s, &lo, &hi);
     }
     if (hi <= lo) {
       for (int c = lane; c < dc; c += 64) orow[c] = 0.f;
       continue;
     }
-    const int64_t cf = lo / p.chunk_len, cl = (hi - 1) / p.chunk_len;
+    const int64_t cf = lo / len, cl = (hi - 1) / len;
     float M = -INFINITY;
     for (int64_t c = cf; c <= cl; ++c) M = fmaxf(M, p.part_lse[(c + s) * p.Hq + hq]);
     float wsum = 0.f;

@@ -81,7 +81,7 @@ struct DecodeProblem {
   int dc, dR, dv;
   float scale_log2;       // softmax scale * log2(e)
   // plan
-  int chunk_len;
+  int chunk_len;       // rows per chunk, or < 0: the filled rows divided on the device (below)
   int num_chunks;
   int num_slots;
   float* part_o;       // fp32 rows O / l, or (part_f16) fp16 rows, see below
@@ -214,6 +214,158 @@ __device__ inline void block_coords(int num_chunks, int groups, int* chunk, int*
 __device__ inline int find_seq_mfma(const DecodeProblem& p, int64_t r) {
   if (p.offsets) return find_seq(p, r);
   return (int)((uint32_t)r / (uint32_t)p.seq_len);
+}
+
+// Chunks over filled rows (chunk_len < 0; MFMA attention kernels with
+// per-sequence lengths and no chunk_rows override). Regions are capacity: cut
+// like the other plans' row space, the chunks over unfilled rows leave their
+// workgroups idle and the others with a longer piece each (16 sequences of 300
+// to 6000 rows in 6016-row regions, FP8, 128 heads: attention
+// 36.4 us against 29.7).
+// Instead every sequence is cut into pieces of its own of at most L rows, and
+// piece c (counted over the sequences) is chunk c of a row space in which each
+// sequence is padded to a multiple of L (filled_piece: at most num_chunks
+// pieces), and no workgroup has a second segment (pieces across sequences, at
+// their mean length, made the step 8 us slower: a segment's fixed part is that
+// of eight tiles). The lengths are on the device, so every wave of the
+// attention kernel sums them itself (wave-uniform code, all lanes active), and
+// its workgroups leave what the merge needs behind the log-sum-exps
+// (filled_notes): summed again there, behind its weight loads, it cost 1.5 us.
+// The lane index is made in an asm statement at each use: held in a register
+// for later segments it would spill beside the 128-head kernel's operands.
+__device__ inline int wave_lane() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
+// Inclusive sum over the lanes (DPP row shifts and broadcasts: no lane index).
+__device__ inline int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+__device__ inline int wave_sum_i(int v) { return __builtin_amdgcn_readlane(wave_scan(v), 63); }
+__device__ inline int filled_rows(const DecodeProblem& p, int s) {
+  return (int)max(seq_end(p, s) - seq_begin(p, s), (int64_t)0);
+}
+__device__ inline int pieces(int rows, int len) { return (int)(((uint32_t)rows + (uint32_t)len - 1) / (uint32_t)len); }
+// Piece c: its sequence (num_seqs if there is none), that sequence's rows and
+// first piece, and L, the fewest rows (a multiple of 32, at least -chunk_len)
+// that num_chunks pieces suffice for: T / num_chunks at best,
+// T / (num_chunks - num_seqs) always. The first 64 lengths stay in registers.
+struct FilledPiece {
+  int s, rows, first, len;
+};
+__device__ inline FilledPiece filled_piece(const DecodeProblem& p, int c) {
+  const int lane = wave_lane();
+  const int mine = lane < p.num_seqs ? filled_rows(p, lane) : 0;
+  int t = mine;
+  for (int i = lane + 64; i < p.num_seqs; i += 64) t += filled_rows(p, i);
+  const uint32_t total = (uint32_t)wave_sum_i(t);
+  auto share = [&](uint32_t n) { return max(-p.chunk_len, (int)(((total + n - 1) / n + 31) & ~31u)); };
+  auto fits = [&](int len) {
+    int n = pieces(mine, len);
+    for (int i = lane + 64; i < p.num_seqs; i += 64) n += pieces(filled_rows(p, i), len);
+    return wave_sum_i(n) <= p.num_chunks;
+  };
+  int lo = share((uint32_t)p.num_chunks), hi = share((uint32_t)(p.num_chunks - p.num_seqs));
+  if (lo != hi && fits(lo)) hi = lo;  // equal sequences take one try
+  else lo = min(lo + 32, hi);
+  while (lo < hi) {
+    const int mid = (lo + hi) / 2 & ~31;  // lo <= mid < hi
+    if (fits(mid)) hi = mid;
+    else lo = mid + 32;
+  }
+  FilledPiece f{p.num_seqs, 0, 0, hi};
+  for (int s0 = 0; s0 < p.num_seqs; s0 += 64) {
+    const int rows = s0 == 0 ? mine : s0 + lane < p.num_seqs ? filled_rows(p, s0 + lane) : 0;
+    const int n = pieces(rows, hi), end = wave_scan(n);
+    const uint64_t past = __builtin_amdgcn_ballot_w64(f.first + end > c);
+    if (past) {
+      const int k = __builtin_ctzll(past);
+      f.s = s0 + k;
+      f.rows = __builtin_amdgcn_readlane(rows, k);
+      f.first += __builtin_amdgcn_readlane(end, k) - __builtin_amdgcn_readlane(n, k);
+      break;
+    }
+    f.first += __builtin_amdgcn_readlane(end, 63);
+  }
+  return f;
+}
+// First chunk of every sequence with rows, then L, written by the attention
+// kernel's first workgroup of each sequence and of the launch.
+__host__ __device__ inline int32_t* filled_notes(const DecodeProblem& p) {
+  return reinterpret_cast<int32_t*>(p.part_lse + (int64_t)p.num_slots * p.Hq);
+}
+// A walk over the segments of one chunk (pieces of it inside one sequence).
+// kFilled: chunk_len may be < 0 (a kernel without it keeps that code, and the
+// registers it holds for later segments, out of its way to the first copy).
+template <bool kFilled>
+struct ChunkWalk {
+  int64_t lo, hi;  // what is left of the chunk, in the plan's row space
+  int s;           // sequence of the current segment
+  int64_t row0;    // first row of that sequence in the cache (its region)
+  int64_t s_lo;    // and in the plan's row space
+  int64_t seg_hi;  // end of the current segment there
+};
+template <bool kFilled>
+__device__ inline bool walk_begin(const DecodeProblem& p, int chunk, int group, ChunkWalk<kFilled>& w) {
+  if (kFilled && p.chunk_len < 0) {
+    const FilledPiece f = filled_piece(p, chunk);
+    if (f.s >= p.num_seqs) return false;
+    w.s = f.s;
+    w.s_lo = (int64_t)f.first * f.len;
+    w.row0 = seq_begin(p, f.s);
+    w.lo = (int64_t)chunk * f.len;
+    w.hi = w.seg_hi = min(w.lo + f.len, w.s_lo + f.rows);
+    if (group == 0 && chunk == f.first) filled_notes(p)[f.s] = f.first;  // the same from every lane
+    if (group == 0 && chunk == 0) filled_notes(p)[p.num_seqs] = f.len;
+    return true;
+  }
+  const int64_t end_all = seq_begin(p, p.num_seqs);
+  w.lo = (int64_t)chunk * p.chunk_len;
+  w.hi = min(w.lo + (int64_t)p.chunk_len, end_all);
+  w.lo = max(w.lo, seq_begin(p, 0));
+  if (w.lo >= w.hi) return false;
+  w.s = find_seq_mfma(p, w.lo);
+  return true;
+}
+// The next segment [lo, seg_hi) of sequence s; after it the caller sets lo = seg_hi and ++s.
+template <bool kFilled>
+__device__ inline bool walk_next(const DecodeProblem& p, ChunkWalk<kFilled>& w) {
+  while (w.lo < w.hi) {
+    if (kFilled && p.chunk_len < 0) return true;  // the one segment, set by walk_begin
+    w.s_lo = w.row0 = seq_begin(p, w.s);
+    w.lo = max(w.lo, w.s_lo);  // past the unfilled rows of the previous region
+    if (w.lo >= w.hi) return false;
+    const int64_t s_hi = seq_end(p, w.s);
+    if (s_hi <= w.lo) {  // empty sequence, or lo in its unfilled rows
+      if (++w.s >= p.num_seqs) return false;
+      continue;
+    }
+    w.seg_hi = min(w.hi, s_hi);
+    return true;
+  }
+  return false;
+}
+
+// Rows [lo, hi) of sequence s in the plan's row space, and the rows per chunk.
+__device__ inline int seq_in_plan(const DecodeProblem& p, int s, int64_t* lo, int64_t* hi) {
+  if (p.chunk_len < 0) {
+    *hi = *lo = 0;
+    if (filled_rows(p, s) == 0) return 1;
+    const int len = filled_notes(p)[p.num_seqs];
+    *lo = (int64_t)filled_notes(p)[s] * len;
+    *hi = *lo + filled_rows(p, s);
+    return len;
+  }
+  *lo = seq_begin(p, s);
+  *hi = seq_end(p, s);
+  return p.chunk_len;
 }
 
 // OCP FP8 E4M3 (e4m3fn) latent-cache element: sign, 4 exponent bits (bias

@@ -949,8 +949,9 @@ static_assert(fp8_half_order_ok(), "fp8 expansion halves overlap");
 
 // kFp8: FP8 E4M3 cache rows (KT = bf16: the tiles are expanded to bf16 in
 // LDS and the MFMAs run on bf16).
-template <typename KT, bool kPaged, bool kFp8>
-__global__ __launch_bounds__(kThreads) void decode_mfma_kernel(DecodeProblem p, int groups) {
+// kFilled: chunks over filled rows (ChunkWalk).
+template <typename KT, bool kPaged, bool kFp8, bool kFilled>
+__device__ __forceinline__ void decode_mfma_body(const DecodeProblem& p, int groups) {
   static_assert(!kFp8 || std::is_same<KT, __hip_bfloat16>::value, "fp8 tiles expand to bf16");
   constexpr int kDma = dma_per_wave(kFp8);
   typedef Ops<KT> O_;
@@ -971,27 +972,15 @@ __global__ __launch_bounds__(kThreads) void decode_mfma_kernel(DecodeProblem p, 
   if (chunk >= p.num_chunks) return;
   const int hg_heads = min(kHG, p.Hq - group * kHG);
 
-  const int64_t end_all = seq_begin(p, p.num_seqs);
-  int64_t lo = (int64_t)chunk * p.chunk_len;
-  const int64_t hi = min(lo + (int64_t)p.chunk_len, end_all);
-  lo = max(lo, seq_begin(p, 0));
-  if (lo >= hi) return;
-  int s = find_seq_mfma(p, lo);
+  ChunkWalk<kFilled> w;
+  if (!walk_begin(p, chunk, group, w)) return;
 
-  while (lo < hi) {
-    const int64_t s_lo = seq_begin(p, s);
-    lo = max(lo, s_lo);  // past the unfilled rows of the previous region
-    if (lo >= hi) break;
-    const int64_t s_hi = seq_end(p, s);
-    if (s_hi <= lo) {  // empty sequence, or lo in its unfilled rows
-      if (++s >= p.num_seqs) break;
-      continue;
-    }
-    const int64_t seg_hi = min(hi, s_hi);
+  while (walk_next(p, w)) {
+    const int s = w.s;
     SegCtx sg;
-    sg.base = reinterpret_cast<const char*>(p.kv) + (kPaged ? 0 : lo * cache_row_bytes<kFp8>());
-    sg.pos0 = lo - s_lo;
-    sg.last = (int)(seg_hi - lo - 1);
+    sg.base = reinterpret_cast<const char*>(p.kv) + (kPaged ? 0 : (w.row0 + (w.lo - w.s_lo)) * cache_row_bytes<kFp8>());
+    sg.pos0 = w.lo - w.s_lo;
+    sg.last = (int)(w.seg_hi - w.lo - 1);
     sg.seq = s;
     sg.tab = kPaged ? p.block_table + (int64_t)s * p.blocks_per_seq : nullptr;
     sg.tile0 = (uint32_t)(sg.pos0 / kT);
@@ -1676,8 +1665,8 @@ __global__ __launch_bounds__(kThreads) void decode_mfma_kernel(DecodeProblem p, 
     asm volatile("" : "+v"(xb[8]), "+v"(xb[9]), "+v"(xb[10]), "+v"(xb[11]), "+v"(xb[12]), "+v"(xb[13]), "+v"(xb[14]), "+v"(xb[15]));
     store16(par, xb);
     LA_STAMP(9);
-    lo = seg_hi;
-    ++s;
+    w.lo = w.seg_hi;
+    ++w.s;
   }
 #ifdef LA_PHASE_STAMPS
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1685,6 +1674,16 @@ __global__ __launch_bounds__(kThreads) void decode_mfma_kernel(DecodeProblem p, 
   if ((threadIdx.x & 63) == 0 && blockIdx.x < kStampBlocks)
     for (int i = 0; i < kStampSlots; ++i) g_attn_stamps[((size_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kStampSlots + i] = stamps_[i];
 #endif
+}
+
+template <typename KT, bool kPaged, bool kFp8>
+__global__ __launch_bounds__(kThreads) void decode_mfma_kernel(DecodeProblem p, int groups) {
+  decode_mfma_body<KT, kPaged, kFp8, kPaged>(p, groups);  // a paged cache always has lengths
+}
+// Contiguous capacity caches: the same with chunks over their filled rows.
+template <typename KT, bool kFp8>
+__global__ __launch_bounds__(kThreads) void decode_mfma_filled_kernel(DecodeProblem p, int groups) {
+  decode_mfma_body<KT, false, kFp8, true>(p, groups);
 }
 
 // Copies-only variant of the attention kernel, for measuring the streaming
@@ -1794,30 +1793,33 @@ __global__ __launch_bounds__(256) void prep_q_kernel(const float* __restrict__ q
   *reinterpret_cast<vec*>(out + qprep_index(qrow, 8 * j)) = v;
 }
 
-template <typename KT, bool kPaged, bool kFp8 = false>
-hipError_t launch_t(const DecodeProblem& p, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
-  static bool attr_set = false;  // per instance; setting it twice is harmless
-  if (!attr_set) {
-    const void* fn = reinterpret_cast<const void*>(&decode_mfma_kernel<KT, kPaged, kFp8>);
+hipError_t launch_k(void (*k)(DecodeProblem, int), bool* attr_set, const DecodeProblem& p, hipStream_t stream,
+                    hipEvent_t ev_begin, hipEvent_t ev_end) {
+  if (!*attr_set) {  // per kernel; setting it twice is harmless
+    const void* fn = reinterpret_cast<const void*>(k);
     hipFuncAttributes fa;
     hipError_t e = hipFuncGetAttributes(&fa, fn);
     if (e != hipSuccess) return e;
     if (fa.sharedSizeBytes != 0) return hipErrorInvalidKernelFile;  // LDS offsets would not be addresses
     e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     if (e != hipSuccess) return e;
-    attr_set = true;
+    *attr_set = true;
   }
   const int groups = (p.Hq + kHG - 1) / kHG;
-  const int64_t blocks = mfma_grid_blocks(p.num_chunks, groups);
-  if (ev_begin || ev_end) {
-    // the events time this kernel's execution alone (no dispatch gap)
-    hipExtLaunchKernelGGL((decode_mfma_kernel<KT, kPaged, kFp8>), dim3((unsigned)blocks), dim3(kThreads), kLdsBytes,
-                          stream, ev_begin, ev_end, 0, p, groups);
-  } else {
-    hipLaunchKernelGGL((decode_mfma_kernel<KT, kPaged, kFp8>), dim3((unsigned)blocks), dim3(kThreads), kLdsBytes, stream,
-                       p, groups);
-  }
+  const dim3 blocks((unsigned)mfma_grid_blocks(p.num_chunks, groups));
+  if (ev_begin || ev_end)  // the events time this kernel's execution alone (no dispatch gap)
+    hipExtLaunchKernelGGL(k, blocks, dim3(kThreads), kLdsBytes, stream, ev_begin, ev_end, 0, p, groups);
+  else
+    hipLaunchKernelGGL(k, blocks, dim3(kThreads), kLdsBytes, stream, p, groups);
   return hipGetLastError();
+}
+
+template <typename KT, bool kFp8>
+hipError_t launch_t(const DecodeProblem& p, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
+  static bool set[3] = {false, false, false};
+  if (p.block_table) return launch_k(decode_mfma_kernel<KT, true, kFp8>, &set[0], p, stream, ev_begin, ev_end);
+  if (p.chunk_len < 0) return launch_k(decode_mfma_filled_kernel<KT, kFp8>, &set[1], p, stream, ev_begin, ev_end);
+  return launch_k(decode_mfma_kernel<KT, false, kFp8>, &set[2], p, stream, ev_begin, ev_end);
 }
 
 }  // namespace
@@ -1890,12 +1892,7 @@ hipError_t launch_stream_copies(const DecodeProblem& p, int ring, hipStream_t st
 }
 
 hipError_t launch_decode_mfma(const DecodeProblem& p, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
-  if (p.block_table) {
-    if (p.kv_dtype == LA_DTYPE_FP8_E4M3) return launch_t<__hip_bfloat16, true, true>(p, stream, ev_begin, ev_end);
-    if (p.kv_dtype == LA_DTYPE_BF16) return launch_t<__hip_bfloat16, true>(p, stream, ev_begin, ev_end);
-    return launch_t<__half, true>(p, stream, ev_begin, ev_end);
-  }
-  if (p.kv_dtype == LA_DTYPE_FP8_E4M3) return launch_t<__hip_bfloat16, false, true>(p, stream, ev_begin, ev_end);
+  if (p.kv_dtype == LA_DTYPE_FP8_E4M3) return launch_t<__hip_bfloat16, true>(p, stream, ev_begin, ev_end);
   if (p.kv_dtype == LA_DTYPE_BF16) return launch_t<__hip_bfloat16, false>(p, stream, ev_begin, ev_end);
   return launch_t<__half, false>(p, stream, ev_begin, ev_end);
 }

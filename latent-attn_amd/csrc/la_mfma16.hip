@@ -166,7 +166,7 @@ __device__ inline float sum_groups(float x) {
 // slower than with the launch.) kW = 4 has no room for it (its k_rope and P rows
 // are smaller than the queries). zero_out (optional): zero_n floats zeroed for
 // a half-row merge.
-template <typename KT, int kW, bool kPaged, bool kFp8>
+template <typename KT, int kW, bool kPaged, bool kFp8, bool kFilled>
 __global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem p, int groups, float* zero_out,
                                                                   int zero_n) {
   typedef Ops16<KT> O_;
@@ -194,26 +194,14 @@ __global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem
   if (chunk >= p.num_chunks) return;
   const int head0 = group * 16;  // Hq is a multiple of 16 (mfma_supported)
 
-  const int64_t end_all = seq_begin(p, p.num_seqs);
-  int64_t lo = (int64_t)chunk * p.chunk_len;
-  const int64_t hi = min(lo + (int64_t)p.chunk_len, end_all);
-  lo = max(lo, seq_begin(p, 0));
-  if (lo >= hi) return;
-  int s = find_seq_mfma(p, lo);
+  ChunkWalk<kFilled> w;
+  if (!walk_begin(p, chunk, group, w)) return;
 
-  while (lo < hi) {
-    const int64_t s_lo = seq_begin(p, s);
-    lo = max(lo, s_lo);  // past the unfilled rows of the previous region
-    if (lo >= hi) break;
-    const int64_t s_hi = seq_end(p, s);
-    if (s_hi <= lo) {  // empty sequence, or lo in its unfilled rows
-      if (++s >= p.num_seqs) break;
-      continue;
-    }
-    const int64_t seg_hi = min(hi, s_hi);
-    const char* const seg_base = reinterpret_cast<const char*>(p.kv) + (kPaged ? 0 : lo * kRowB);
-    const uint32_t pos0 = (uint32_t)(lo - s_lo);
-    const int last = (int)(seg_hi - lo - 1);
+  while (walk_next(p, w)) {
+    const int s = w.s;
+    const char* const seg_base = reinterpret_cast<const char*>(p.kv) + (kPaged ? 0 : (w.row0 + (w.lo - w.s_lo)) * kRowB);
+    const uint32_t pos0 = (uint32_t)(w.lo - w.s_lo);
+    const int last = (int)(w.seg_hi - w.lo - 1);
     const int ntiles = last / kT + 1;
     const int rlim = p.rope_rows > 0 ? (int)(p.rope_rows - 1) : INT32_MAX;
 
@@ -490,18 +478,18 @@ __global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem
       *reinterpret_cast<i16x8*>(dst + head * (kDc * 2)) = lds_ld<i16x8>(L, head * D::kStagePitch + 16 * lane);
     }
     lds_barrier();  // the staging is read before the next segment's tile lands on it
-    lo = seg_hi;
-    ++s;
+    w.lo = w.seg_hi;
+    ++w.s;
   }
 }
 
-template <typename KT, int kW, bool kPaged, bool kFp8>
+template <typename KT, int kW, bool kPaged, bool kFp8, bool kFilled>
 hipError_t launch16_t(const DecodeProblem& p, hipStream_t stream, float* zero_out, int zero_n, hipEvent_t ev_begin,
                       hipEvent_t ev_end) {
   constexpr int lds = Lds<kW>::kBytes;
   static bool attr_set = false;  // per instance; setting it twice is harmless
   if (!attr_set) {
-    const void* fn = reinterpret_cast<const void*>(&decode_mfma16_kernel<KT, kW, kPaged, kFp8>);
+    const void* fn = reinterpret_cast<const void*>(&decode_mfma16_kernel<KT, kW, kPaged, kFp8, kFilled>);
     const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return e;
     attr_set = true;
@@ -509,26 +497,31 @@ hipError_t launch16_t(const DecodeProblem& p, hipStream_t stream, float* zero_ou
   const int groups = p.Hq / 16;
   const dim3 grid((unsigned)mfma_grid_blocks(p.num_chunks, groups));
   if (ev_begin || ev_end)
-    hipExtLaunchKernelGGL((decode_mfma16_kernel<KT, kW, kPaged, kFp8>), grid, dim3(64 * kW), lds, stream, ev_begin,
+    hipExtLaunchKernelGGL((decode_mfma16_kernel<KT, kW, kPaged, kFp8, kFilled>), grid, dim3(64 * kW), lds, stream, ev_begin,
                           ev_end, 0, p, groups, zero_out, zero_n);
   else
-    hipLaunchKernelGGL((decode_mfma16_kernel<KT, kW, kPaged, kFp8>), grid, dim3(64 * kW), lds, stream, p, groups, zero_out,
+    hipLaunchKernelGGL((decode_mfma16_kernel<KT, kW, kPaged, kFp8, kFilled>), grid, dim3(64 * kW), lds, stream, p, groups, zero_out,
                        zero_n);
   return hipGetLastError();
 }
 
-template <int kW>
+template <int kW, bool kPaged, bool kFilled>
 hipError_t launch16_w(const DecodeProblem& p, hipStream_t stream, float* zero_out, int zero_n, hipEvent_t ev_begin,
                       hipEvent_t ev_end) {
   typedef __hip_bfloat16 B;
-  if (p.block_table) {
-    if (p.kv_dtype == LA_DTYPE_FP8_E4M3) return launch16_t<B, kW, true, true>(p, stream, zero_out, zero_n, ev_begin, ev_end);
-    if (p.kv_dtype == LA_DTYPE_BF16) return launch16_t<B, kW, true, false>(p, stream, zero_out, zero_n, ev_begin, ev_end);
-    return launch16_t<__half, kW, true, false>(p, stream, zero_out, zero_n, ev_begin, ev_end);
-  }
-  if (p.kv_dtype == LA_DTYPE_FP8_E4M3) return launch16_t<B, kW, false, true>(p, stream, zero_out, zero_n, ev_begin, ev_end);
-  if (p.kv_dtype == LA_DTYPE_BF16) return launch16_t<B, kW, false, false>(p, stream, zero_out, zero_n, ev_begin, ev_end);
-  return launch16_t<__half, kW, false, false>(p, stream, zero_out, zero_n, ev_begin, ev_end);
+  if (p.kv_dtype == LA_DTYPE_FP8_E4M3)
+    return launch16_t<B, kW, kPaged, true, kFilled>(p, stream, zero_out, zero_n, ev_begin, ev_end);
+  if (p.kv_dtype == LA_DTYPE_BF16)
+    return launch16_t<B, kW, kPaged, false, kFilled>(p, stream, zero_out, zero_n, ev_begin, ev_end);
+  return launch16_t<__half, kW, kPaged, false, kFilled>(p, stream, zero_out, zero_n, ev_begin, ev_end);
+}
+
+template <int kW>
+hipError_t launch16_k(const DecodeProblem& p, hipStream_t stream, float* zero_out, int zero_n, hipEvent_t ev_begin,
+                      hipEvent_t ev_end) {
+  if (p.block_table) return launch16_w<kW, true, true>(p, stream, zero_out, zero_n, ev_begin, ev_end);
+  if (p.chunk_len < 0) return launch16_w<kW, false, true>(p, stream, zero_out, zero_n, ev_begin, ev_end);
+  return launch16_w<kW, false, false>(p, stream, zero_out, zero_n, ev_begin, ev_end);
 }
 
 }  // namespace
@@ -536,8 +529,8 @@ hipError_t launch16_w(const DecodeProblem& p, hipStream_t stream, float* zero_ou
 hipError_t launch_decode_mfma16(const DecodeProblem& p, int waves, hipStream_t stream, float* zero_out, int64_t zero_n,
                                 hipEvent_t ev_begin, hipEvent_t ev_end) {
   if (zero_n > INT32_MAX / 2) return hipErrorInvalidValue;  // the kernel counts in 32 bits
-  return waves == 8 ? launch16_w<8>(p, stream, zero_out, (int)zero_n, ev_begin, ev_end)
-                    : launch16_w<4>(p, stream, zero_out, (int)zero_n, ev_begin, ev_end);
+  return waves == 8 ? launch16_k<8>(p, stream, zero_out, (int)zero_n, ev_begin, ev_end)
+                    : launch16_k<4>(p, stream, zero_out, (int)zero_n, ev_begin, ev_end);
 }
 
 }  // namespace la

@@ -399,10 +399,11 @@ __device__ inline MergeTask merge_task(const DecodeProblem& p, int t, int h, int
   if (t < 0 || t >= p.num_seqs * p.qps) return m;
   const int s = t / p.qps;
   const int hq = (t % p.qps) * p.nh + h;
-  const int64_t lo = seq_begin(p, s), hi = seq_end(p, s);
+  int64_t lo, hi;
+  const int len = seq_in_plan(p, s, &lo, &hi);
   if (hi <= lo) return m;
-  const int64_t cf = lo / p.chunk_len;
-  m.n = (int)((hi - 1) / p.chunk_len - cf + 1);  // slots cf+s .. cf+s+n-1
+  const int64_t cf = lo / len;
+  m.n = (int)((hi - 1) / len - cf + 1);  // slots cf+s .. cf+s+n-1
   m.ns = m.n > g ? (m.n - g + G - 1) / G : 0;
   m.row0 = (cf + s) * p.Hq + hq;
   return m;
@@ -522,11 +523,11 @@ __device__ inline void merge_tasks(const DecodeProblem& p, const int (&t)[kTasks
 // so its 128 KB of W_UV is fetched once per head.
 constexpr int kMPWaves = 8;
 // slot rows each task loads up front (one memory round trip for up to this
-// many; more loop over further batches, a round trip each). The half-row
-// merge also comes with 32 (8 B per lane each), launched when a task has
-// more than 16 slots (4 rows of 64 slots: 32 a task, 14.9 us against 19.5): its
-// 205 VGPRs leave one workgroup per CU, where 108 leave two (16 slots a task,
-// 16 rows: 18.4 us against 13.6).
+// many; more loop over further batches, a round trip each). The half-row merge
+// also comes with 16 and 32 (8 B per lane each), taken by the slots per task:
+// 8 / 16 / 32 at once take 14.5 / 13.9 / 18.7 us for 16 slots, 18.9 / 19.6 /
+// 15.6 for 32, 5.9 / 6.0 / 6.4 for one (88, 104 and 136 VGPRs: fewer
+// workgroups per CU).
 constexpr int kMPSlots = 8;
 constexpr int kMPPitch = kDcP + 4;  // floats per LDS row of a slot-group sum
 // 16-bit elements per LDS row of the high / low operand rows: 1040 B, 16 B
@@ -904,18 +905,20 @@ hipError_t launch_combine_project_mfma(const DecodeProblem& p, hipStream_t strea
     while (rpb_log2 > 0 && hb * ((R + (1 << rpb_log2) - 1) >> rpb_log2) < ncu) --rpb_log2;
     const int rpb = 1 << rpb_log2;
     const dim3 grid((unsigned)(hb * ((R + rpb - 1) >> rpb_log2)));
-    // slots per task with equal sequences (seq_len / chunk_len when chunks
-    // align with the sequences, else up to two more; rows of a block share
-    // G = 8 / rows tasks); ragged or capacity caches keep the 8-slot batches
+    // Slots per row: seq_len / chunk_len with equal sequences whose chunks align
+    // with them, else up to two more; a sequence's share of the chunks where
+    // the lengths are on the device. The rows of a block share G = 8 / rows
+    // tasks, which load 8, 16 or 32 slots at once (kMPSlots).
     const int G = kMPWaves / (R < rpb ? R : rpb);
-    const int64_t n = p.offsets || p.lens || p.chunk_len <= 0 ? 0
-                      : p.seq_len % p.chunk_len == 0 ? p.seq_len / p.chunk_len
-                                                     : p.seq_len / p.chunk_len + 2;
-    const bool wide = (n + G - 1) / G > 2 * kMPSlots;
-    auto k = p.wuv_dtype == LA_DTYPE_BF16 ? (wide ? merge_project_half_kernel<__hip_bfloat16, 32>
-                                                  : merge_project_half_kernel<__hip_bfloat16, kMPSlots>)
-                                          : (wide ? merge_project_half_kernel<__half, 32>
-                                                  : merge_project_half_kernel<__half, kMPSlots>);
+    const int64_t n = p.offsets || p.lens || p.chunk_len <= 0 ? p.num_chunks / p.num_seqs
+                      : p.seq_len % p.chunk_len == 0          ? p.seq_len / p.chunk_len
+                                                              : p.seq_len / p.chunk_len + 2;
+    const int64_t per = (n + G - 1) / G;
+    const bool bf = p.wuv_dtype == LA_DTYPE_BF16;
+    auto k = per > 16 ? (bf ? merge_project_half_kernel<__hip_bfloat16, 32> : merge_project_half_kernel<__half, 32>)
+             : per > kMPSlots ? (bf ? merge_project_half_kernel<__hip_bfloat16, 16> : merge_project_half_kernel<__half, 16>)
+                              : (bf ? merge_project_half_kernel<__hip_bfloat16, kMPSlots>
+                                    : merge_project_half_kernel<__half, kMPSlots>);
     hipLaunchKernelGGL(k, grid, dim3(kMPWaves * 64), 0, stream, p, rpb_log2);
     return hipGetLastError();
   }

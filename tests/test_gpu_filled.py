@@ -1,0 +1,61 @@
+"""Decode with per-sequence lengths: the MFMA kernels' chunks share the filled
+rows, found on the device (seq_in_plan / ChunkWalk, csrc/la_internal.hpp).
+More sequences than a wave has lanes, empty ones, lengths around the padding
+of 32, one long sequence among short ones, over capacity, packed and paged
+caches, against the float64 oracle over the filled rows; unfilled rows hold
+values that would dominate any softmax."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import assert_close
+from mla_cases import TORCH_DTYPE, cfg_with_heads, make_queries, make_weights, rope, to_np
+from oracle import mla_oracle as mo
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("layout", ["capacity", "packed", "paged"])
+@pytest.mark.parametrize("dtype,heads", [("bf16", 128), ("f16", 16), ("fp8", 128), ("f32", 16)])
+@pytest.mark.parametrize("lens", [[0, 31, 32, 33, 1, 0, 200] + [5, 64] * 33, [0] * 3, [3000, 1, 40]])
+def test_filled_rows(cuda, layout, dtype, heads, lens):
+    from latent_attn import functional as F
+
+    cfg = cfg_with_heads(heads)
+    B, bs = len(lens), 32
+    cap = 224 if max(lens) <= 200 else 3008
+    wt = {"fp8": "bf16"}.get(dtype, dtype)
+    dt = torch.float8_e4m3fn if dtype == "fp8" else TORCH_DTYPE[dtype]
+    W_UK, W_UV = make_weights(cfg, wt, 3, cuda)
+    q_nope, q_rope = make_queries((B,), cfg, 4, cuda)
+    cos, sin = rope(cap, cfg, cuda)
+    g = torch.Generator().manual_seed(5)
+    seqs = [torch.randn(n, 576, generator=g).to(dt) for n in lens]
+    rows = torch.full((B * cap, 576), 96.0).to(dt).view(torch.uint8)
+    for b, s in enumerate(seqs):
+        rows[b * cap:b * cap + len(s)] = s.view(torch.uint8)
+    len_t = torch.tensor(lens, dtype=torch.int32, device=cuda)
+    args = (q_nope, q_rope, W_UK, W_UV, cos, sin, cfg)
+    if layout == "capacity":
+        out = F.mla_decode(rows.view(dt).to(cuda).view(B, cap, 576), *args, seq_lens=len_t)
+    elif layout == "packed":
+        off = torch.arange(B + 1, dtype=torch.int32, device=cuda) * cap
+        out = F.mla_decode(rows.view(dt).to(cuda), *args, seq_offsets=off, seq_lens=len_t)
+    else:
+        table = torch.randperm(B * cap // bs, generator=g)
+        pool = torch.empty_like(rows).view(-1, bs, rows.size(1))
+        pool[table] = rows.view(-1, bs, rows.size(1))
+        out = F.mla_decode(pool.view(-1, rows.size(1)).view(dt).to(cuda), *args, seq_lens=len_t,
+                           block_table=table.to(torch.int32).view(B, -1).to(cuda), block_size=bs)
+    d = mo.Dims(cfg.d_model, 512, 128, 64, heads, 128)
+    qa = mo.absorb_q(to_np(q_nope), to_np(W_UK), d)
+    off_np = np.concatenate([[0], np.cumsum(lens)]).tolist()
+    packed = np.concatenate([to_np(s).reshape(-1, 576) for s in seqs])
+    ref = mo.decode_sequences(packed, off_np, qa, to_np(q_rope), to_np(W_UV), to_np(cos), to_np(sin), d)
+    if not any(lens):
+        assert torch.count_nonzero(out).item() == 0
+        return
+    assert_close(out.cpu().numpy(), ref, wt, f"filled {layout} {dtype} H={heads} B={B}")
