@@ -357,10 +357,13 @@ __device__ inline bool walk_next(const DecodeProblem& p, ChunkWalk<kFilled>& w) 
 __device__ inline int seq_in_plan(const DecodeProblem& p, int s, int64_t* lo, int64_t* hi) {
   if (p.chunk_len < 0) {
     *hi = *lo = 0;
-    if (filled_rows(p, s) == 0) return 1;
-    const int len = filled_notes(p)[p.num_seqs];
-    *lo = (int64_t)filled_notes(p)[s] * len;
-    *hi = *lo + filled_rows(p, s);
+    const int rows = filled_rows(p, s);
+    if (rows == 0) return 1;
+    // clamped into the plan: malformed offsets can leave notes unwritten (their
+    // row sum wraps), which gives wrong answers but no access out of bounds
+    const int len = max(filled_notes(p)[p.num_seqs], 1);
+    *lo = (int64_t)min(max(filled_notes(p)[s], 0), p.num_chunks - 1) * len;
+    *hi = min(*lo + rows, (int64_t)p.num_chunks * len);
     return len;
   }
   *lo = seq_begin(p, s);
