@@ -553,11 +553,12 @@ size_t la_fused_mla_workspace_size_dt(int seq_len, int batch_size, const la_mla_
                                       int w_uv_dtype) {
   if (!cfg || seq_len < 0 || batch_size <= 0) return 0;
   // Only plan-relevant fields are read. Which kernel family runs also depends
-  // on pointer alignment, so return the larger of the two families' plans.
+  // on pointer alignment, so return the largest of the families' plans (the
+  // fp32 MFMA kernel has no variant of its own: 0 plans it).
   alignas(256) static const char dummy[256] = {0};
   const float* d = reinterpret_cast<const float*>(dummy);
   size_t best = 0;
-  for (int variant : {1, 2}) {
+  for (int variant : {0, 1, 2}) {
     la_decode_args a = la::shared_cache_args(dummy, kv_dtype, seq_len, batch_size, d, d, dummy, w_uv_dtype, d, d,
                                              const_cast<float*>(d), cfg, nullptr, 0);
     a.kernel_variant = variant;

@@ -36,8 +36,8 @@
 // kernel -> this one: 1 x 512, 128 heads, fp16 16.2 -> 7.9 (kW = 8; 9.6 with
 // 4); 1 x 8192, 128 heads 17.0 -> 11.6 (15.4 with 8); 32 x 4099 with 16 heads
 // 51.3 -> 33.4, with 32 heads 52.2 -> 38.0; with 64 heads 52.7 -> 60.2 and 16
-// queries over 2048 rows 21.7 -> 36.3 (both stay on the 128-head kernel,
-// mfma16_waves). Two head blocks per workgroup (Q and O fill the registers)
+// queries over 2048 rows 21.7 -> 36.3 (both stay on the 128-head kernel: the
+// plan's waves16). Two head blocks per workgroup (Q and O fill the registers)
 // took 45.7 at 32 heads and 50.2 at 64.
 #include "la_internal.hpp"
 

@@ -83,3 +83,24 @@ def test_absorb(cuda, tokens, dn):
     got = F.absorb_q(q.to(cuda), W.to(cuda), cfg)
     ref = np.einsum("thi,hic->thc", to_np(q), to_np(W).reshape(3, dn, 512))
     assert_close(got.cpu().numpy(), ref, "f32", f"absorb f32 tokens {tokens} dn {dn}")
+
+
+@pytest.mark.parametrize("seq,heads", [(2048, 128), (4099, 16)])
+def test_shared_cache_workspace(cuda, seq, heads):
+    """The shared-cache entry points size their workspace for the fp32 kernel's chunks (more than the VALU kernel's)."""
+    from latent_attn import functional as F
+
+    cfg = cfg_with_heads(heads)
+    _, W_UV = make_weights(cfg, "f32", 9, cuda)
+    cos, sin = rope(seq, cfg, cuda)
+    g = torch.Generator().manual_seed(10)
+    kv = torch.randn(seq, 576, generator=g).to(cuda)
+    qa = torch.randn(2, heads, 512, generator=g).to(cuda)
+    qr = torch.randn(2, heads, 64, generator=g).to(cuda)
+    out = F.batched_fused_mla(kv, qa, qr, W_UV, cos, sin, cfg).cpu().numpy()
+    one = F.fused_mla(kv, qa[1], qr[1], W_UV, cos, sin, cfg).cpu().numpy()
+    args = [to_np(x) for x in (W_UV, cos, sin)]
+    for b in range(2):
+        ref = mo.decode_sequences(to_np(kv), [0, seq], to_np(qa[b])[None], to_np(qr[b])[None], *args, _dims(cfg))
+        assert_close(out[b][None], ref, "f32", f"f32 shared cache S={seq} H={heads} query {b}")
+    assert_close(one[None], ref, "f32", f"f32 fused S={seq} H={heads}")
