@@ -289,9 +289,10 @@ int la_stream_ceiling(const la_decode_args* args, int32_t ring, void* stream, vo
  * step needs (16-bit queries, split partials) comes from a static device
  * array of la_mla_decode_noalloc_max_bytes() bytes (64 MiB) that each GPU the
  * library runs on holds until the process ends; args->workspace and
- * workspace_bytes are ignored. Steps needing more than that return
- * LA_ERROR_WORKSPACE before any device work (la_mla_decode_workspace_size
- * gives the need). Every call on one GPU shares that GPU's array: calls that
+ * workspace_bytes are ignored. A step whose plan needs more than that
+ * (la_mla_decode_workspace_size) is cut into fewer chunks where its kernel
+ * has such a plan (float32 caches, up to 32 query heads, seq_lens); if that
+ * needs more too, it returns LA_ERROR_WORKSPACE before any device work. Every call on one GPU shares that GPU's array: calls that
  * overlap on one GPU (two streams, two threads) race and must be serialised
  * by the caller. Nothing in the array needs to start at zero; it keeps the
  * last call's contents. */

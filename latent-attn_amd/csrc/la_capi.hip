@@ -70,7 +70,10 @@ struct Plan {
 
 // Fills the problem (without workspace pointers) and the plan. The args'
 // chunk_rows / kernel_variant fields are tuning overrides (0 = automatic).
-int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
+// coarse: the chunks of one 128-head (or VALU) workgroup per target block, also
+// for the kernels with 16 heads per workgroup, and no plan over filled rows:
+// fewer partial slots, for a caller whose scratch does not hold the others.
+int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse = false) {
   if (!a || !valid_cfg(&a->cfg)) return LA_ERROR_INVALID_VALUE;
   const int chunk_rows = a->chunk_rows;
   const int variant = a->kernel_variant;
@@ -160,7 +163,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
   int64_t L, min_rows = 64;
   if (chunk_rows > 0) {
     L = chunk_rows;
-  } else if (pl.f32) {
+  } else if (pl.f32 && !coarse) {
     // two workgroups per CU, but no chunks under 128 rows while one per CU
     // remains: their partial rows (2 KB per head) cost the merge more than the
     // second workgroup gains (4 x 1000 rows, 128 heads: 51.5 us a step against
@@ -170,7 +173,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
     L = std::max<int64_t>(((total + chunks - 1) / chunks + 15) / 16 * 16, 64);
     if (L < 128 && groups * ((total + 127) / 128) >= ncu) L = 128;
     min_rows = std::min<int64_t>(L, 128);
-  } else if (few_heads) {
+  } else if (few_heads && !coarse) {
     // two workgroups per CU and no more (16 heads x 131168 rows: 33.4 us with
     // 257-row chunks, 37 with 128, 35.6 with 513); whole tiles only where a
     // paged cache needs them, so that rounding leaves no CU without a chunk
@@ -241,7 +244,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan) {
     off += align_up((size_t)pl.num_slots * p->Hq * 3 * sizeof(float));
   }
   pl.part_lse_off = off;
-  const bool filled = a->seq_lens && chunk_rows == 0 && (pl.mfma || pl.f32) && 4LL * a->num_seqs <= nchunks &&
+  const bool filled = !coarse && a->seq_lens && chunk_rows == 0 && (pl.mfma || pl.f32) && 4LL * a->num_seqs <= nchunks &&
                       total <= INT32_MAX;
   off += align_up((size_t)pl.num_slots * p->Hq * sizeof(float) +
                   (filled ? ((size_t)a->num_seqs + 1) * sizeof(int32_t) : 0));  // filled_notes
@@ -278,11 +281,11 @@ bool merge_halves(const DecodeProblem& p, const Plan& plan) {
 // ev_b / ev_e (optional) are recorded around the attention kernel, which runs
 // max(repeat, 1) times between them.
 int run(const la_decode_args* a, hipStream_t stream, hipEvent_t ev_b = nullptr, hipEvent_t ev_e = nullptr,
-        int repeat = 1) {
+        int repeat = 1, bool coarse = false) {
   if (repeat < 0) return LA_ERROR_INVALID_VALUE;
   DecodeProblem p;
   Plan plan;
-  int st = prepare(a, &p, &plan);
+  int st = prepare(a, &p, &plan, coarse);
   if (st != LA_SUCCESS) return st;
   if (a->num_seqs == 0) return LA_SUCCESS;
 
@@ -515,7 +518,9 @@ int la_stream_ceiling(const la_decode_args* args, int32_t ring, void* stream, vo
 int la_mla_decode_noalloc(const la_decode_args* args, void* stream) {
   la::DecodeProblem p;
   la::Plan plan;
-  const int st = la::prepare(args, &p, &plan);
+  int st = la::prepare(args, &p, &plan);
+  const bool coarse = st == LA_SUCCESS && plan.total > la::kNoAllocScratchBytes;
+  if (coarse) st = la::prepare(args, &p, &plan, true);
   if (st != LA_SUCCESS) return st;
   if (plan.total > la::kNoAllocScratchBytes) return LA_ERROR_WORKSPACE;
   la_decode_args a = *args;
@@ -525,7 +530,7 @@ int la_mla_decode_noalloc(const la_decode_args* args, void* stream) {
     const int sp = la::scratch_ptr(&a.workspace);
     if (sp != LA_SUCCESS) return sp;
   }  // else: no workspace is needed and none is passed
-  return la::run(&a, static_cast<hipStream_t>(stream));
+  return la::run(&a, static_cast<hipStream_t>(stream), nullptr, nullptr, 1, coarse);
 }
 
 size_t la_mla_decode_noalloc_max_bytes(void) { return la::kNoAllocScratchBytes; }

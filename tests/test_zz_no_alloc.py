@@ -18,7 +18,7 @@ import numpy as np
 import pytest
 import torch
 
-from mla_cases import make_cache, make_queries, make_weights, rope
+from mla_cases import cfg_with_heads, make_cache, make_queries, make_weights, rope
 
 from latent_attn import MLAConfig, capi
 
@@ -146,3 +146,49 @@ def test_noalloc_under_hip_graph_capture(cuda):
         print(f"[noalloc] replay {r}", flush=True)
         assert torch.equal(out, want), (r, float((out - want).abs().max()))
         assert torch.equal(other, want)
+
+
+@pytest.mark.parametrize("dtype,heads", [("f32", 128), ("bf16", 16), ("bf16", 32)])
+def test_noalloc_cuts_fewer_chunks_at_the_scratch_limit(cuda, dtype, heads):
+    """The first batch whose plan no longer fits the scratch still runs, on fewer chunks: the same
+    output as with a workspace up to the order of the merge's sums."""
+    lib = capi.load()
+    cfg = cfg_with_heads(heads)
+    S = 64
+    code = {"f32": capi.LA_DTYPE_F32, "bf16": capi.LA_DTYPE_BF16}[dtype]
+    W_UK, W_UV = make_weights(cfg, dtype, 211, cuda)
+    cos, sin = rope(S, cfg, cuda)
+
+    def args(kv, q_nope, q_rope, out):
+        a = _args(kv, None, S, q_nope, q_rope, W_UK, W_UV, cos, sin, out, cfg)
+        a.kv_dtype = a.w_uk_dtype = a.w_uv_dtype = code
+        return a
+
+    a = args(torch.empty(1, 576, dtype=W_UK.dtype, device=cuda), *[torch.empty(1, device=cuda)] * 3)
+    most = lib.la_mla_decode_noalloc_max_bytes()
+    for B in range(32, 4096):
+        a.num_seqs, a.total_rows = B, B * S
+        if lib.la_mla_decode_workspace_size(ctypes.byref(a)) > most:
+            break
+    else:
+        pytest.fail("no batch exceeds the scratch")
+    kv = make_cache((B * S,), cfg, dtype, 212, cuda)
+    q_nope, q_rope = make_queries((B,), cfg, 213, cuda)
+    out = torch.empty(B, heads, 128, device=cuda)
+    a = args(kv, q_nope, q_rope, out)
+    need = lib.la_mla_decode_workspace_size(ctypes.byref(a))
+    assert need > most
+    ws = torch.empty(need, dtype=torch.uint8, device=cuda)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), need
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert lib.la_mla_decode(ctypes.byref(a), stream) == capi.LA_SUCCESS
+    torch.cuda.synchronize()
+    want = out.clone()
+    out.fill_(float("nan"))
+    a.workspace, a.workspace_bytes = None, 0
+    st = lib.la_mla_decode_noalloc(ctypes.byref(a), stream)
+    assert st == capi.LA_SUCCESS, lib.la_status_string(st)
+    torch.cuda.synchronize()
+    # fp32 partials differ by their sums' order; fp16 partial rows by their rounding, 2^-11 of a row's largest
+    rel = float((out - want).norm() / want.norm())
+    assert rel < (2e-6 if dtype == "f32" else 2e-3), rel
