@@ -291,7 +291,7 @@ int la_stream_ceiling(const la_decode_args* args, int32_t ring, void* stream, vo
  * library runs on holds until the process ends; args->workspace and
  * workspace_bytes are ignored. A step whose plan needs more than that
  * (la_mla_decode_workspace_size) is cut into fewer chunks where its kernel
- * has such a plan (float32 caches, up to 32 query heads, seq_lens); if that
+ * has such a plan (float32 caches, up to 32 query heads); if that
  * needs more too, it returns LA_ERROR_WORKSPACE before any device work. Every call on one GPU shares that GPU's array: calls that
  * overlap on one GPU (two streams, two threads) race and must be serialised
  * by the caller. Nothing in the array needs to start at zero; it keeps the

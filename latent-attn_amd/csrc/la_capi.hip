@@ -71,8 +71,7 @@ struct Plan {
 // Fills the problem (without workspace pointers) and the plan. The args'
 // chunk_rows / kernel_variant fields are tuning overrides (0 = automatic).
 // coarse: the chunks of one 128-head (or VALU) workgroup per target block, also
-// for the kernels with 16 heads per workgroup, and no plan over filled rows:
-// fewer partial slots, for a caller whose scratch does not hold the others.
+// for the kernels with 16 heads per workgroup: fewer partial slots, for a caller whose scratch does not hold the others.
 int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse = false) {
   if (!a || !valid_cfg(&a->cfg)) return LA_ERROR_INVALID_VALUE;
   const int chunk_rows = a->chunk_rows;
@@ -244,10 +243,9 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
     off += align_up((size_t)pl.num_slots * p->Hq * 3 * sizeof(float));
   }
   pl.part_lse_off = off;
-  const bool filled = !coarse && a->seq_lens && chunk_rows == 0 && (pl.mfma || pl.f32) && 4LL * a->num_seqs <= nchunks &&
+  const bool filled = a->seq_lens && chunk_rows == 0 && (pl.mfma || pl.f32) && 4LL * a->num_seqs <= nchunks &&
                       total <= INT32_MAX;
-  off += align_up((size_t)pl.num_slots * p->Hq * sizeof(float) +
-                  (filled ? ((size_t)a->num_seqs + 1) * sizeof(int32_t) : 0));  // filled_notes
+  off += align_up((size_t)pl.num_slots * p->Hq * sizeof(float));
   pl.proj_mfma = project_mfma_supported(*p);
   pl.proj_f32 = project_f32_supported(*p);
   pl.total = off;

@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kThreads, 2) void decode_f32_kernel(DecodeProblem p
 #pragma unroll
       for (int c = 0; c < 4; ++c) settle(o[cb][c]);
     if (head0 + n16 < p.Hq) {
-      const int64_t row = ((int64_t)chunk + s) * p.Hq + head0 + n16;
+      const int64_t row = (kFilled ? slot_of(p, chunk, s) : (int64_t)chunk + s) * p.Hq + head0 + n16;
       const float inv = 1.f / l;
       // accumulator (cb, c), element r: column 128 wave + 64 cb + 4 (4 g + r) + c
       float* dst = p.part_o + row * kDc + 128 * wave + 16 * g;

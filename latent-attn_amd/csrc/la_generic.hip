@@ -184,11 +184,11 @@ __global__ __launch_bounds__(kCombineThreads) void combine_project_kernel(Decode
     }
     const int64_t cf = lo / len, cl = (hi - 1) / len;
     float M = -INFINITY;
-    for (int64_t c = cf; c <= cl; ++c) M = fmaxf(M, p.part_lse[(c + s) * p.Hq + hq]);
+    for (int64_t c = cf; c <= cl; ++c) M = fmaxf(M, p.part_lse[slot_of(p, c, s) * p.Hq + hq]);
     float wsum = 0.f;
     for (int c = lane; c < dc; c += 64) orow[c] = 0.f;
     for (int64_t c = cf; c <= cl; ++c) {
-      const int64_t slot = c + s;
+      const int64_t slot = slot_of(p, c, s);
       const float w = exp2f(p.part_lse[slot * p.Hq + hq] - M);
       wsum += w;
       const int64_t prow = slot * p.Hq + hq;

@@ -229,7 +229,7 @@ __device__ inline int find_seq_mfma(const DecodeProblem& p, int64_t r) {
 // their mean length, made the step 8 us slower: a segment's fixed part is that
 // of eight tiles). The lengths are on the device, so every wave of the
 // attention kernel sums them itself (wave-uniform code, all lanes active), and
-// its workgroups leave what the merge needs behind the log-sum-exps
+// its workgroups leave what the merge needs in free slots
 // (filled_notes): summed again there, behind its weight loads, it cost 1.5 us.
 // The lane index is made in an asm statement at each use: held in a register
 // for later segments it would spill beside the 128-head kernel's operands.
@@ -297,10 +297,17 @@ __device__ inline FilledPiece filled_piece(const DecodeProblem& p, int c) {
   return f;
 }
 // First chunk of every sequence with rows, then L, written by the attention
-// kernel's first workgroup of each sequence and of the launch.
-__host__ __device__ inline int32_t* filled_notes(const DecodeProblem& p) {
-  return reinterpret_cast<int32_t*>(p.part_lse + (int64_t)p.num_slots * p.Hq);
+// kernel's first workgroup of each sequence and of the launch. A piece lies in
+// one sequence, so chunk c writes slot c and the num_seqs - 1 slots after the
+// chunks' are free: the notes (num_seqs + 1 words) take their partial rows (at
+// least 1 KB each), and the workspace is that of the other plans. One sequence
+// has no free slot and needs no notes: seq_in_plan divides its rows itself.
+__device__ inline int32_t* filled_notes(const DecodeProblem& p) {
+  return reinterpret_cast<int32_t*>(reinterpret_cast<char*>(p.part_o) +
+                                    (int64_t)p.num_chunks * p.Hq * p.dc * (p.part_f16 ? 2 : 4));
 }
+// Partial slot of the piece of chunk c inside sequence s.
+__device__ inline int64_t slot_of(const DecodeProblem& p, int64_t c, int s) { return c + (p.chunk_len < 0 ? 0 : s); }
 // A walk over the segments of one chunk (pieces of it inside one sequence).
 // kFilled: chunk_len may be < 0 (a kernel without it keeps that code, and the
 // registers it holds for later segments, out of its way to the first copy).
@@ -322,8 +329,10 @@ __device__ inline bool walk_begin(const DecodeProblem& p, int chunk, int group, 
     w.row0 = seq_begin(p, f.s);
     w.lo = (int64_t)chunk * f.len;
     w.hi = w.seg_hi = min(w.lo + f.len, w.s_lo + f.rows);
-    if (group == 0 && chunk == f.first) filled_notes(p)[f.s] = f.first;  // the same from every lane
-    if (group == 0 && chunk == 0) filled_notes(p)[p.num_seqs] = f.len;
+    if (p.num_seqs > 1 && group == 0) {  // the same from every lane
+      if (chunk == f.first) filled_notes(p)[f.s] = f.first;
+      if (chunk == 0) filled_notes(p)[p.num_seqs] = f.len;
+    }
     return true;
   }
   const int64_t end_all = seq_begin(p, p.num_seqs);
@@ -359,6 +368,11 @@ __device__ inline int seq_in_plan(const DecodeProblem& p, int s, int64_t* lo, in
     *hi = *lo = 0;
     const int rows = filled_rows(p, s);
     if (rows == 0) return 1;
+    if (p.num_seqs == 1) {  // as filled_piece: num_chunks pieces always suffice
+      const uint32_t n = (uint32_t)p.num_chunks;
+      *hi = rows;
+      return max(-p.chunk_len, (int)((((uint32_t)rows + n - 1) / n + 31) & ~31u));
+    }
     // clamped into the plan: malformed offsets can leave notes unwritten (their
     // row sum wraps), which gives wrong answers but no access out of bounds
     const int len = max(filled_notes(p)[p.num_seqs], 1);

@@ -1554,7 +1554,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeProblem& p, int gro
     const int le = lane_id();  // fresh: the prologue's lane index would come back from a spill slot
     const int g2 = le >> 5;
     const float l_tot = sum_halves(l_run);
-    const int64_t slot = (int64_t)chunk + s;
+    const int64_t slot = kFilled ? slot_of(p, chunk, s) : (int64_t)chunk + s;
     const int64_t hqg = slot * p.Hq + group * kHG;  // slot row of head 0 of the group
     if (le < 32 && 32 * wave + le < hg_heads) {
       p.part_lse[hqg + 32 * wave + le] = m_run + log2f(l_tot);

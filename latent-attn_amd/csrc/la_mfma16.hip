@@ -431,7 +431,7 @@ __global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem
     lds_barrier();  // every wave is done with the tile
     const int lane = fresh_lane();
     const int n16 = lane & 15, g = lane >> 4;
-    const int64_t hq0 = ((int64_t)chunk + s) * p.Hq + head0;
+    const int64_t hq0 = (kFilled ? slot_of(p, chunk, s) : (int64_t)chunk + s) * p.Hq + head0;
     float rmax = 0.f;
 #pragma unroll
     for (int cb = 0; cb < kCB; ++cb) settle(o[cb]);

@@ -403,9 +403,9 @@ __device__ inline MergeTask merge_task(const DecodeProblem& p, int t, int h, int
   const int len = seq_in_plan(p, s, &lo, &hi);
   if (hi <= lo) return m;
   const int64_t cf = lo / len;
-  m.n = (int)((hi - 1) / len - cf + 1);  // slots cf+s .. cf+s+n-1
+  m.n = (int)((hi - 1) / len - cf + 1);  // slots slot_of(cf) .. + n - 1
   m.ns = m.n > g ? (m.n - g + G - 1) / G : 0;
-  m.row0 = (cf + s) * p.Hq + hq;
+  m.row0 = slot_of(p, cf, s) * p.Hq + hq;
   return m;
 }
 

@@ -20,7 +20,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("layout", ["capacity", "packed", "paged"])
 @pytest.mark.parametrize("dtype,heads", [("bf16", 128), ("f16", 16), ("fp8", 128), ("f32", 16)])
-@pytest.mark.parametrize("lens", [[0, 31, 32, 33, 1, 0, 200] + [5, 64] * 33, [0] * 3, [3000, 1, 40]])
+@pytest.mark.parametrize("lens", [[0, 31, 32, 33, 1, 0, 200] + [5, 64] * 33, [0] * 3, [3000, 1, 40], [2001]])
 def test_filled_rows(cuda, layout, dtype, heads, lens):
     from latent_attn import functional as F
 
@@ -59,3 +59,25 @@ def test_filled_rows(cuda, layout, dtype, heads, lens):
         assert torch.count_nonzero(out).item() == 0
         return
     assert_close(out.cpu().numpy(), ref, wt, f"filled {layout} {dtype} H={heads} B={B}")
+
+
+@pytest.mark.parametrize("heads,dtype", [(128, "bf16"), (16, "bf16"), (128, "f32")])
+def test_workspace_serves_a_batch_with_and_without_lengths(cuda, heads, dtype):
+    """A workspace sized for whole regions holds the same batch with lengths, contiguous and paged (host only)."""
+    import ctypes
+
+    from latent_attn import capi
+
+    lib = capi.load()
+    a = capi.DecodeArgs()
+    fake = 0x10000
+    code = {"bf16": capi.LA_DTYPE_BF16, "f32": capi.LA_DTYPE_F32}[dtype]
+    a.kv_cache = a.q_nope = a.W_UK = a.q_rope = a.W_UV = a.rope_cos = a.rope_sin = a.output = fake
+    a.kv_dtype = a.w_uk_dtype = a.w_uv_dtype = code
+    a.num_seqs, a.seq_len, a.queries_per_seq, a.total_rows = 32, 8192, 1, 32 * 8192
+    a.cfg = capi.config(cfg_with_heads(heads))
+    whole = lib.la_mla_decode_workspace_size(ctypes.byref(a))
+    a.seq_lens = fake
+    assert 0 < lib.la_mla_decode_workspace_size(ctypes.byref(a)) <= whole
+    a.seq_len, a.block_table, a.block_size, a.blocks_per_seq = 0, fake, 64, 128
+    assert 0 < lib.la_mla_decode_workspace_size(ctypes.byref(a)) <= whole
