@@ -235,7 +235,8 @@ enum {
   LA_PLAN_MERGE_VALU = 1,        /* combine_project_kernel */
   LA_PLAN_MERGE_MFMA = 2,        /* merge_project_kernel: full partial rows per workgroup */
   LA_PLAN_MERGE_MFMA_HALVES = 3, /* merge_project_half_kernel: latent halves added into the output */
-  LA_PLAN_MERGE_MFMA_F32 = 4     /* merge_project_f32_kernel: float32 weights */
+  LA_PLAN_MERGE_MFMA_F32 = 4,    /* merge_project_f32_kernel: float32 weights */
+  LA_PLAN_MERGE_MFMA_F32_HALVES = 5 /* the same over latent halves added into the output */
 };
 enum {
   LA_PLAN_ABSORB_NONE = 0,       /* queries come absorbed (q_absorbed) */
@@ -249,10 +250,13 @@ typedef struct la_plan_info {
   int32_t chunk_rows;  /* rows per split-KV chunk (of the regions; shorter on the device with seq_lens) */
   int32_t num_chunks;
   int32_t num_slots;   /* partial slots per query head: num_chunks + num_seqs - 1 */
-  int32_t head_groups; /* groups of 128 query heads per chunk (one workgroup each, or eight where the plan's
-                          16-head MFMA kernel runs; the launch is rounded for the XCDs) */
+  int32_t head_groups; /* groups of query heads per chunk: of 128 (LA_PLAN_ATTENTION_MFMA), of 16 (_MFMA_F32) or of
+                          one (_VALU) */
   int32_t merge;       /* LA_PLAN_MERGE_* */
   int32_t absorb;      /* LA_PLAN_ABSORB_* */
+  int16_t heads_per_workgroup; /* query heads of one attention workgroup: 1 (VALU), 128 (decode_mfma_kernel) or 16
+                          (decode_mfma16_kernel, decode_f32_kernel); a chunk has ceil(query heads / it) of them */
+  int16_t filled_rows; /* 1: the chunks are pieces of the sequences' filled rows, cut on the device (seq_lens) */
   size_t workspace_bytes; /* la_mla_decode_workspace_size(args) */
 } la_plan_info;
 int la_mla_decode_plan(const la_decode_args* args, la_plan_info* info);

@@ -462,6 +462,8 @@ size_t la_mla_decode_workspace_size(const la_decode_args* args) {
   return plan.total;
 }
 
+static_assert(sizeof(la_plan_info) == 32 + sizeof(size_t) && offsetof(la_plan_info, workspace_bytes) == 32,
+              "the layout of callers built against seven 32-bit fields");
 int la_mla_decode_plan(const la_decode_args* args, la_plan_info* info) {
   if (!info) return LA_ERROR_INVALID_VALUE;
   la::DecodeProblem p;
@@ -475,8 +477,11 @@ int la_mla_decode_plan(const la_decode_args* args, la_plan_info* info) {
   info->chunk_rows = plan.chunk_len;
   info->num_chunks = plan.num_chunks;
   info->num_slots = plan.num_slots;
-  info->head_groups = plan.mfma ? (p.Hq + la::mfma_heads_per_group() - 1) / la::mfma_heads_per_group() : p.Hq;
-  if (plan.proj_f32) info->merge = LA_PLAN_MERGE_MFMA_F32;
+  const int group = plan.mfma ? la::mfma_heads_per_group() : plan.f32 ? 16 : 1;
+  info->head_groups = (p.Hq + group - 1) / group;
+  info->heads_per_workgroup = (int16_t)(plan.waves16 ? 16 : group);
+  info->filled_rows = p.chunk_len < 0;
+  if (plan.proj_f32) info->merge = la::merge_halves(p, plan) ? LA_PLAN_MERGE_MFMA_F32_HALVES : LA_PLAN_MERGE_MFMA_F32;
   else if (!plan.proj_mfma) info->merge = LA_PLAN_MERGE_VALU;
   else info->merge = la::merge_halves(p, plan) ? LA_PLAN_MERGE_MFMA_HALVES : LA_PLAN_MERGE_MFMA;
   if (!args->q_nope) info->absorb = LA_PLAN_ABSORB_NONE;

@@ -94,13 +94,17 @@ class PlanInfo(ctypes.Structure):
         ("head_groups", ctypes.c_int32),
         ("merge", ctypes.c_int32),
         ("absorb", ctypes.c_int32),
+        ("heads_per_workgroup", ctypes.c_int16),
+        ("filled_rows", ctypes.c_int16),
         ("workspace_bytes", ctypes.c_size_t),
     ]
 
 
-LA_PLAN_ATTENTION_VALU, LA_PLAN_ATTENTION_MFMA = 1, 2
+LA_PLAN_ATTENTION_VALU, LA_PLAN_ATTENTION_MFMA, LA_PLAN_ATTENTION_MFMA_F32 = 1, 2, 3
 LA_PLAN_MERGE_VALU, LA_PLAN_MERGE_MFMA, LA_PLAN_MERGE_MFMA_HALVES = 1, 2, 3
+LA_PLAN_MERGE_MFMA_F32, LA_PLAN_MERGE_MFMA_F32_HALVES = 4, 5
 LA_PLAN_ABSORB_NONE, LA_PLAN_ABSORB_VALU, LA_PLAN_ABSORB_MFMA, LA_PLAN_ABSORB_MFMA_QPREP = 0, 1, 2, 3
+LA_PLAN_ABSORB_MFMA_F32 = 4
 
 _lib = None
 

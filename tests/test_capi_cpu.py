@@ -192,6 +192,16 @@ def test_plan_query_without_a_gfx950_device():
     assert lib.la_mla_decode_plan(ctypes.byref(a), None) == capi.LA_ERROR_INVALID_VALUE
 
 
+def test_plan_info_layout():
+    """The fields that tell the kernels apart lie where la_plan_info had padding: its size and the
+    offsets of the others are those of callers built before them."""
+    i = capi.PlanInfo
+    assert ctypes.sizeof(i) == 40 and i.absorb.offset == 24 and i.workspace_bytes.offset == 32
+    lib, info = capi.load(), capi.PlanInfo()
+    assert lib.la_mla_decode_plan(ctypes.byref(_args()), ctypes.byref(info)) == capi.LA_SUCCESS
+    assert (info.heads_per_workgroup, info.filled_rows) == (1, 0)  # the VALU kernel, on this host
+
+
 def test_stream_ceiling_rejects_bad_arguments():
     """la_stream_ceiling (the copies-only measurement of the attention
     kernel's copy schedule) checks its ring depth, repeat count and

@@ -1,0 +1,63 @@
+"""The plan that la_mla_decode_plan reports, kernel by kernel (host only: no
+pointer is read). Tests of one kernel assert through it that their sizes reach
+that kernel."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+
+from mla_cases import cfg_with_heads
+
+from latent_attn import capi
+
+pytestmark = pytest.mark.gpu
+
+CODE = {"bf16": capi.LA_DTYPE_BF16, "f16": capi.LA_DTYPE_F16, "f32": capi.LA_DTYPE_F32, "fp8": capi.LA_DTYPE_FP8_E4M3}
+
+
+def plan_args(dtype, heads, num_seqs, seq_len, qps=1, wdtype=None, **kw):
+    a = capi.DecodeArgs()
+    fake = 0x10000
+    a.kv_cache = a.q_nope = a.W_UK = a.q_rope = a.W_UV = a.rope_cos = a.rope_sin = a.output = fake
+    a.kv_dtype = CODE[dtype]
+    a.w_uk_dtype = a.w_uv_dtype = CODE[wdtype or {"fp8": "bf16"}.get(dtype, dtype)]
+    a.num_seqs, a.seq_len, a.queries_per_seq, a.total_rows = num_seqs, seq_len, qps, num_seqs * seq_len
+    a.cfg = capi.config(cfg_with_heads(heads))
+    for k, v in kw.items():
+        setattr(a, k, v)
+    return a
+
+
+def plan(*args, **kw):
+    a, info = plan_args(*args, **kw), capi.PlanInfo()
+    assert capi.load().la_mla_decode_plan(ctypes.byref(a), ctypes.byref(info)) == capi.LA_SUCCESS
+    return info
+
+
+# (dtype, heads, sequences, rows, queries, other fields): attention, head_groups, heads_per_workgroup, filled_rows, merge
+MFMA, F32, VALU = capi.LA_PLAN_ATTENTION_MFMA, capi.LA_PLAN_ATTENTION_MFMA_F32, capi.LA_PLAN_ATTENTION_VALU
+LENS = {"seq_lens": 0x10000}
+
+
+@pytest.mark.parametrize("args,kw,want", [
+    (("bf16", 128, 1, 512), {}, (MFMA, 1, 16, 0, capi.LA_PLAN_MERGE_MFMA_HALVES)),
+    (("bf16", 128, 32, 8192), {}, (MFMA, 1, 128, 0, capi.LA_PLAN_MERGE_MFMA)),
+    (("f16", 48, 1, 16384, 3), {}, (MFMA, 2, 128, 0, capi.LA_PLAN_MERGE_MFMA_HALVES)),
+    (("fp8", 16, 32, 4099), {}, (MFMA, 1, 16, 0, capi.LA_PLAN_MERGE_MFMA_HALVES)),
+    (("fp8", 128, 16, 6016), LENS, (MFMA, 1, 128, 1, capi.LA_PLAN_MERGE_MFMA_HALVES)),
+    (("bf16", 128, 16, 6016), {**LENS, "chunk_rows": 512}, (MFMA, 1, 128, 0, capi.LA_PLAN_MERGE_MFMA_HALVES)),
+    (("f32", 128, 4, 1000), {}, (F32, 8, 16, 0, capi.LA_PLAN_MERGE_MFMA_F32_HALVES)),
+    (("f32", 20, 64, 1000), {}, (F32, 2, 16, 0, capi.LA_PLAN_MERGE_MFMA_F32_HALVES)),
+    (("f32", 128, 32, 100), {}, (F32, 8, 16, 0, capi.LA_PLAN_MERGE_MFMA_F32)),
+    (("f32", 128, 4, 1000), {"kernel_variant": 1}, (VALU, 128, 1, 0, capi.LA_PLAN_MERGE_MFMA_F32)),
+])
+def test_plan_names_the_kernels(cuda, args, kw, want):
+    import torch
+
+    if torch.cuda.get_device_properties(cuda).multi_processor_count != 256:
+        pytest.skip("the sizes are of 256 CUs")
+    i = plan(*args, **kw)
+    assert (i.attention, i.head_groups, i.heads_per_workgroup, i.filled_rows, i.merge) == want
+    assert i.absorb == (capi.LA_PLAN_ABSORB_MFMA_F32 if args[0] == "f32" else capi.LA_PLAN_ABSORB_MFMA_QPREP)
