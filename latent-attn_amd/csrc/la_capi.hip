@@ -204,7 +204,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
     L = std::max<int64_t>(L, 64);
   }
   if (L > (int64_t)1 << 30) L = (int64_t)1 << 30;
-  if ((pl.mfma || pl.f32) && L > mfma_max_chunk_rows()) L = mfma_max_chunk_rows();
+  if ((pl.mfma || pl.f32) && L > kMaxChunkRows) L = kMaxChunkRows;
   if (paged && (pl.mfma || pl.f32)) L = (L + 63) / 64 * 64;  // MFMA tiles start block-aligned
   const int64_t nchunks = total > 0 ? (total + L - 1) / L : 0;
   if (nchunks > (int64_t)1 << 30) return LA_ERROR_INVALID_VALUE;
@@ -243,8 +243,10 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
     off += align_up((size_t)pl.num_slots * p->Hq * 3 * sizeof(float));
   }
   pl.part_lse_off = off;
+  const int piece = (int)std::min<int64_t>((min_rows + 31) / 32 * 32, L);  // shortest piece of filled rows
   const bool filled = a->seq_lens && chunk_rows == 0 && (pl.mfma || pl.f32) && 4LL * a->num_seqs <= nchunks &&
-                      total <= INT32_MAX;
+                      total <= INT32_MAX &&
+                      piece_rows((uint32_t)total, (uint32_t)(nchunks - a->num_seqs), piece) <= kMaxChunkRows;
   off += align_up((size_t)pl.num_slots * p->Hq * sizeof(float));
   pl.proj_mfma = project_mfma_supported(*p);
   pl.proj_f32 = project_f32_supported(*p);
@@ -257,8 +259,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
   // uneven pieces: 165 us a step against 147 over their 4096-row regions; 64 of
   // 300 to 8192: 120 against 154; 32 of 500 to 8000 in 32768-row regions: 74
   // against 208).
-  if (filled)
-    p->chunk_len = -(int)std::min<int64_t>((min_rows + 31) / 32 * 32, L);
+  if (filled) p->chunk_len = -piece;
   p->num_chunks = pl.num_chunks;
   p->num_slots = pl.num_slots;
   *plan = pl;

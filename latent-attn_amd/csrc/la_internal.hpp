@@ -40,6 +40,9 @@ __host__ __device__ inline int64_t qprep_index(int64_t qrow, int c) {
   return (qrow >> 5) * (32 * kQPrepRow) + 512 * (c >> 4) + 8 * ((qrow & 31) + 32 * ((c >> 3) & 1)) + (c & 7);
 }
 
+// Longest chunk, or piece of filled rows, that the MFMA kernels take: keeps row byte offsets inside 32 bits.
+constexpr int kMaxChunkRows = 1 << 20;
+
 struct DecodeProblem {
   const void* kv;
   int kv_dtype;
@@ -253,6 +256,12 @@ __device__ inline int filled_rows(const DecodeProblem& p, int s) {
   return (int)max(seq_end(p, s) - seq_begin(p, s), (int64_t)0);
 }
 __device__ inline int pieces(int rows, int len) { return (int)(((uint32_t)rows + (uint32_t)len - 1) / (uint32_t)len); }
+// Rows of a piece when n pieces share total rows, at least the plan's shortest. The plan cuts filled rows only
+// where the longest piece of its whole row space is a length that the kernels take.
+__host__ __device__ inline int piece_rows(uint32_t total, uint32_t n, int shortest) {
+  const int rows = (int)(((total + n - 1) / n + 31) & ~31u);
+  return rows > shortest ? rows : shortest;
+}
 // Piece c: its sequence (num_seqs if there is none), that sequence's rows and
 // first piece, and L, the fewest rows (a multiple of 32, at least -chunk_len)
 // that num_chunks pieces suffice for: T / num_chunks at best,
@@ -266,7 +275,8 @@ __device__ inline FilledPiece filled_piece(const DecodeProblem& p, int c) {
   int t = mine;
   for (int i = lane + 64; i < p.num_seqs; i += 64) t += filled_rows(p, i);
   const uint32_t total = (uint32_t)wave_sum_i(t);
-  auto share = [&](uint32_t n) { return max(-p.chunk_len, (int)(((total + n - 1) / n + 31) & ~31u)); };
+  // (malformed offsets can add up to more than the row space: their pieces stay within the kernels' length)
+  auto share = [&](uint32_t n) { return min(piece_rows(total, n, -p.chunk_len), kMaxChunkRows); };
   auto fits = [&](int len) {
     int n = pieces(mine, len);
     for (int i = lane + 64; i < p.num_seqs; i += 64) n += pieces(filled_rows(p, i), len);
@@ -323,7 +333,8 @@ template <bool kFilled>
 __device__ inline bool walk_begin(const DecodeProblem& p, int chunk, int group, ChunkWalk<kFilled>& w) {
   if (kFilled && p.chunk_len < 0) {
     const FilledPiece f = filled_piece(p, chunk);
-    if (f.s >= p.num_seqs) return false;
+    // the last two: malformed offsets, whose sums wrap
+    if (f.s >= p.num_seqs || chunk < f.first || (int64_t)(chunk - f.first) * f.len >= f.rows) return false;
     w.s = f.s;
     w.s_lo = (int64_t)f.first * f.len;
     w.row0 = seq_begin(p, f.s);
@@ -369,9 +380,8 @@ __device__ inline int seq_in_plan(const DecodeProblem& p, int s, int64_t* lo, in
     const int rows = filled_rows(p, s);
     if (rows == 0) return 1;
     if (p.num_seqs == 1) {  // as filled_piece: num_chunks pieces always suffice
-      const uint32_t n = (uint32_t)p.num_chunks;
       *hi = rows;
-      return max(-p.chunk_len, (int)((((uint32_t)rows + n - 1) / n + 31) & ~31u));
+      return piece_rows((uint32_t)rows, (uint32_t)p.num_chunks, -p.chunk_len);
     }
     // clamped into the plan: malformed offsets can leave notes unwritten (their
     // row sum wraps), which gives wrong answers but no access out of bounds
@@ -545,7 +555,6 @@ hipError_t launch_decode_mfma16(const DecodeProblem& p, int waves, hipStream_t s
 // contiguous caches.
 hipError_t launch_stream_copies(const DecodeProblem& p, int ring, hipStream_t stream);
 int mfma_heads_per_group();
-int mfma_max_chunk_rows();
 // Fills p.q_prep from p.q_abs and p.q_rope (MFMA path only).
 // zero_out (optional): zero_n floats zeroed for a latent-half merge.
 hipError_t launch_prep_q(const DecodeProblem& p, hipStream_t stream, float* zero_out = nullptr, int64_t zero_n = 0);

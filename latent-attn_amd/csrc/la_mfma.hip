@@ -220,9 +220,6 @@ constexpr int pv_wait_n(int s, bool fp8) {
 static_assert(pv_wait_n(kExpWaitStep - 1, true) == pv_later(kExpWaitStep - 1) + 4, "fp8 expansion reads counted exactly");
 static_assert(kExpWaitStep > kRotStep && kExpWaitStep + 3 < kPvSteps && kExpSlot0 + 7 < 2 * kPvSteps,
               "fp8 expansion slots inside PV");
-// Longest chunk the kernel accepts: keeps row byte offsets inside 32 bits.
-constexpr int kMaxChunkRows = 1 << 20;
-
 static_assert(kLdsBytes <= 160 * 1024, "LDS budget");
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -1840,7 +1837,6 @@ bool device_is_gfx950() {
 }
 
 int mfma_heads_per_group() { return kHG; }
-int mfma_max_chunk_rows() { return kMaxChunkRows; }
 
 bool mfma_supported(const DecodeProblem& p) {
   if (p.kv_dtype != LA_DTYPE_BF16 && p.kv_dtype != LA_DTYPE_F16 && p.kv_dtype != LA_DTYPE_FP8_E4M3) return false;

@@ -61,3 +61,18 @@ def test_plan_names_the_kernels(cuda, args, kw, want):
     i = plan(*args, **kw)
     assert (i.attention, i.head_groups, i.heads_per_workgroup, i.filled_rows, i.merge) == want
     assert i.absorb == (capi.LA_PLAN_ABSORB_MFMA_F32 if args[0] == "f32" else capi.LA_PLAN_ABSORB_MFMA_QPREP)
+
+
+@pytest.mark.parametrize("heads,num_seqs,seq_len,filled", [
+    (128, 200, 5368704, 0),  # 1,024 chunks of 2^20 rows: 824 pieces would hold 1.24 times that each
+    (128, 16, 67108832, 0),  # 1,008 pieces, still more than 2^20 rows each
+    (128, 32, 1048576, 1),   # 256 chunks of 131,072 rows, pieces of at most 149,824
+])
+def test_filled_pieces_stay_within_the_kernels_chunk_length(cuda, heads, num_seqs, seq_len, filled):
+    """Every sequence full, the pieces of filled rows are up to num_chunks / (num_chunks - num_seqs)
+    times the plan's chunks: a plan whose pieces could pass 2^20 rows keeps its chunks of the regions."""
+    i = plan("fp8", heads, num_seqs, seq_len, rope_rows=8192, **LENS)
+    assert i.attention == MFMA and i.filled_rows == filled and i.num_chunks >= 4 * num_seqs
+    if filled:
+        n = i.num_chunks - num_seqs
+        assert (num_seqs * seq_len + n - 1) // n <= 1 << 20
