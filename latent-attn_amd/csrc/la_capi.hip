@@ -139,6 +139,8 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
   if (a->total_rows > 0 && !a->kv_cache) return LA_ERROR_INVALID_VALUE;
 
   Plan pl;
+  // the fp32 MFMA kernels write and read 16-byte vectors of the workspace
+  const bool ws_aligned = (reinterpret_cast<uintptr_t>(a->workspace) & 15) == 0;
   // An FP8 E4M3 cache runs on the MFMA kernel too (its tiles are expanded to
   // bf16 in LDS); the VALU kernel (kernel_variant 1) reads it as well.
   const bool mfma_ok = mfma_supported(*p);
@@ -146,7 +148,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
   if (variant == kGeneric || !mfma_ok) {
     if (!generic_supported(*p)) return LA_ERROR_NOT_SUPPORTED;
     pl.mfma = false;
-    pl.f32 = variant == kAuto && decode_f32_supported(*p);
+    pl.f32 = variant == kAuto && decode_f32_supported(*p) && ws_aligned;
   } else {
     pl.mfma = true;
   }
@@ -223,7 +225,8 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
   pl.absorb_mfma = absorb && absorb_mfma_supported(a->w_uk_dtype, c.num_heads, c.qk_nope_head_dim, c.kv_lora_rank) &&
                    (reinterpret_cast<uintptr_t>(a->q_nope) & 15) == 0 &&
                    (reinterpret_cast<uintptr_t>(a->W_UK) & 15) == 0;
-  pl.absorb_f32 = absorb && absorb_f32_supported(a->q_nope, a->W_UK, a->w_uk_dtype, c.qk_nope_head_dim, c.kv_lora_rank);
+  pl.absorb_f32 = absorb && absorb_f32_supported(a->q_nope, a->W_UK, a->w_uk_dtype, static_cast<float*>(a->workspace),
+                                                 c.qk_nope_head_dim, c.kv_lora_rank);
   pl.absorb_prep = pl.mfma && pl.absorb_mfma;
   size_t off = 0;
   if (absorb && !pl.absorb_prep) {
@@ -249,7 +252,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
                       piece_rows((uint32_t)total, (uint32_t)(nchunks - a->num_seqs), piece) <= kMaxChunkRows;
   off += align_up((size_t)pl.num_slots * p->Hq * sizeof(float));
   pl.proj_mfma = project_mfma_supported(*p);
-  pl.proj_f32 = project_f32_supported(*p);
+  pl.proj_f32 = project_f32_supported(*p) && ws_aligned;
   pl.total = off;
 
   p->chunk_len = pl.chunk_len;
@@ -703,7 +706,7 @@ int la_absorb_q(const float* q_nope, const void* W_UK, int w_uk_dtype, float* q_
   if (!la::valid_cfg(cfg) || tokens < 0 || !la::valid_dtype(w_uk_dtype)) return LA_ERROR_INVALID_VALUE;
   if (tokens == 0) return LA_SUCCESS;
   if (!q_nope || !W_UK || !q_absorbed) return LA_ERROR_INVALID_VALUE;
-  if (la::absorb_f32_supported(q_nope, W_UK, w_uk_dtype, cfg->qk_nope_head_dim, cfg->kv_lora_rank)) {
+  if (la::absorb_f32_supported(q_nope, W_UK, w_uk_dtype, q_absorbed, cfg->qk_nope_head_dim, cfg->kv_lora_rank)) {
     const hipError_t f = la::launch_absorb_f32(q_nope, W_UK, q_absorbed, tokens, cfg->num_heads, cfg->qk_nope_head_dim,
                                                cfg->kv_lora_rank, static_cast<hipStream_t>(stream));
     return f == hipSuccess ? (int)LA_SUCCESS : la::record_hip(f);

@@ -347,9 +347,10 @@ hipError_t launch_decode_f32(const DecodeProblem& p, hipStream_t stream, float* 
                          : launch_f32_t<false, false>(p, stream, zero_out, zero_n);
 }
 
-bool absorb_f32_supported(const void* q_nope, const void* W, int w_dtype, int dn, int dc) {
-  return w_dtype == LA_DTYPE_F32 && dn % 16 == 0 && dc % 64 == 0 && (reinterpret_cast<uintptr_t>(q_nope) & 15) == 0 &&
-         (reinterpret_cast<uintptr_t>(W) & 15) == 0 && device_is_gfx950();
+bool absorb_f32_supported(const void* q_nope, const void* W, int w_dtype, const float* q_abs, int dn, int dc) {
+  const auto aligned = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+  return w_dtype == LA_DTYPE_F32 && dn % 16 == 0 && dc % 64 == 0 && aligned(q_nope) && aligned(W) && aligned(q_abs) &&
+         device_is_gfx950();
 }
 
 hipError_t launch_absorb_f32(const float* q_nope, const void* W, float* q_abs, int tokens, int nh, int dn, int dc,

@@ -534,7 +534,7 @@ bool device_is_gfx950();
 // (optional): zero_n floats the attention kernel zeroes for a half-row merge.
 bool decode_f32_supported(const DecodeProblem& p);
 hipError_t launch_decode_f32(const DecodeProblem& p, hipStream_t stream, float* zero_out = nullptr, int64_t zero_n = 0);
-bool absorb_f32_supported(const void* q_nope, const void* W_UK, int w_dtype, int dn, int dc);
+bool absorb_f32_supported(const void* q_nope, const void* W_UK, int w_dtype, const float* q_abs, int dn, int dc);
 hipError_t launch_absorb_f32(const float* q_nope, const void* W_UK, float* q_abs, int tokens, int nh, int dn, int dc,
                              hipStream_t stream);
 

@@ -4,6 +4,8 @@ query rows per merge, against the float64 oracle at the fp32 tolerance."""
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -104,3 +106,68 @@ def test_shared_cache_workspace(cuda, seq, heads):
         ref = mo.decode_sequences(to_np(kv), [0, seq], to_np(qa[b])[None], to_np(qr[b])[None], *args, _dims(cfg))
         assert_close(out[b][None], ref, "f32", f"f32 shared cache S={seq} H={heads} query {b}")
     assert_close(one[None], ref, "f32", f"f32 fused S={seq} H={heads}")
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+def test_absorb_into_an_output_that_is_only_float_aligned(cuda, shift):
+    """The MFMA absorption stores 16-byte vectors: an output without that alignment takes the VALU
+    kernel, as a q_nope without it does (the same bits)."""
+    from latent_attn import capi
+
+    lib, cfg = capi.load(), cfg_with_heads(3)
+    g = torch.Generator().manual_seed(11)
+    q = torch.randn(5 * 3 * 128, generator=g).to(cuda)
+    W = torch.randn(3 * 128, 512, generator=g).to(cuda)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def absorb(q_shift, out_shift):
+        buf = torch.empty(q.numel() + 4, device=cuda)
+        buf[q_shift:q_shift + q.numel()] = q
+        out = torch.full((5 * 3 * 512 + 4,), 7.0, device=cuda)
+        c = capi.config(cfg)
+        assert lib.la_absorb_q(buf.data_ptr() + 4 * q_shift, W.data_ptr(), capi.LA_DTYPE_F32,
+                               out.data_ptr() + 4 * out_shift, 5, ctypes.byref(c), stream) == capi.LA_SUCCESS
+        torch.cuda.synchronize()
+        rest = torch.cat([out[:out_shift], out[out_shift + 5 * 3 * 512:]])
+        assert torch.all(rest == 7.0)
+        return out[out_shift:out_shift + 5 * 3 * 512]
+
+    got, valu = absorb(0, shift), absorb(1, 0)
+    assert torch.equal(got, valu) == bool(shift)  # the MFMA kernel sums in another order
+    ref = np.einsum("thi,hic->thc", to_np(q).reshape(5, 3, 128), to_np(W).reshape(3, 128, 512))
+    assert_close(got.cpu().numpy().reshape(5, 3, 512), ref, "f32", f"absorb f32, output shift {shift}")
+
+
+@pytest.mark.parametrize("heads", [1, 16])
+@pytest.mark.parametrize("shift", [0, 4])
+def test_workspace_that_is_only_float_aligned(cuda, heads, shift):
+    """A float32 step over a workspace without 16-byte alignment runs on the VALU kernels."""
+    from latent_attn import capi
+    from test_gpu_plan import F32, VALU
+
+    lib, cfg = capi.load(), cfg_with_heads(heads)
+    B, S = 2, 300
+    W_UK, W_UV = make_weights(cfg, "f32", 3, cuda)
+    q_nope, q_rope = make_queries((B,), cfg, 4, cuda)
+    cos, sin = rope(S, cfg, cuda)
+    kv = torch.randn(B * S, 576, generator=torch.Generator().manual_seed(5)).to(cuda)
+    out = torch.empty(B, heads, 128, device=cuda)
+    a, info = capi.DecodeArgs(), capi.PlanInfo()
+    a.kv_cache, a.kv_dtype, a.total_rows, a.num_seqs, a.seq_len = kv.data_ptr(), capi.LA_DTYPE_F32, B * S, B, S
+    a.queries_per_seq, a.q_nope, a.W_UK, a.q_rope, a.W_UV = 1, q_nope.data_ptr(), W_UK.data_ptr(), q_rope.data_ptr(), W_UV.data_ptr()
+    a.w_uk_dtype = a.w_uv_dtype = capi.LA_DTYPE_F32
+    a.rope_cos, a.rope_sin, a.rope_rows, a.output = cos.data_ptr(), sin.data_ptr(), S, out.data_ptr()
+    a.cfg = capi.config(cfg)
+    a.workspace = 0x10000 + shift
+    assert lib.la_mla_decode_plan(ctypes.byref(a), ctypes.byref(info)) == capi.LA_SUCCESS
+    assert info.attention == (VALU if shift else F32)
+    assert info.absorb == (capi.LA_PLAN_ABSORB_VALU if shift else capi.LA_PLAN_ABSORB_MFMA_F32)
+    assert info.merge == (capi.LA_PLAN_MERGE_VALU if shift else capi.LA_PLAN_MERGE_MFMA_F32_HALVES)
+    ws = torch.empty(info.workspace_bytes + 16, dtype=torch.uint8, device=cuda)
+    a.workspace, a.workspace_bytes = ws.data_ptr() + shift, info.workspace_bytes
+    assert lib.la_mla_decode(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    d = _dims(cfg)
+    ref = mo.decode_sequences(to_np(kv), [0, S, 2 * S], mo.absorb_q(to_np(q_nope), to_np(W_UK), d), to_np(q_rope),
+                              to_np(W_UV), to_np(cos), to_np(sin), d)
+    assert_close(out.cpu().numpy(), ref, "f32", f"f32 H={heads}, workspace + {shift} B")
