@@ -463,7 +463,23 @@ size_t la_mla_decode_workspace_size(const la_decode_args* args) {
   la::DecodeProblem p;
   la::Plan plan;
   if (la::prepare(args, &p, &plan) != LA_SUCCESS) return 0;
-  return plan.total;
+  size_t bytes = plan.total;
+  if (args->num_seqs > 0 && args->kv_dtype == LA_DTYPE_F32 && args->kernel_variant == la::kAuto) {
+    // Alignment alone decides between the two float32 kernels, and either may
+    // take more chunks (one head over 100,000 rows: 782 on the VALU kernel, 481
+    // on the fp32 MFMA kernel): the size serves both, so it does not depend on
+    // the pointers that the step is called with.
+    la_decode_args a = *args;
+    a.kernel_variant = la::kGeneric;
+    if (la::prepare(&a, &p, &plan) == LA_SUCCESS) bytes = std::max(bytes, plan.total);
+    alignas(16) static const float aligned[4] = {0.f};
+    a.kernel_variant = la::kAuto;
+    a.workspace = nullptr;
+    a.kv_cache = a.q_rope = a.rope_cos = a.rope_sin = aligned;
+    if (a.q_absorbed) a.q_absorbed = aligned;
+    if (la::prepare(&a, &p, &plan) == LA_SUCCESS) bytes = std::max(bytes, plan.total);
+  }
+  return bytes;
 }
 
 static_assert(sizeof(la_plan_info) == 32 + sizeof(size_t) && offsetof(la_plan_info, workspace_bytes) == 32,
@@ -475,7 +491,7 @@ int la_mla_decode_plan(const la_decode_args* args, la_plan_info* info) {
   const int st = la::prepare(args, &p, &plan);
   if (st != LA_SUCCESS) return st;
   *info = la_plan_info{};
-  info->workspace_bytes = plan.total;
+  info->workspace_bytes = la_mla_decode_workspace_size(args);
   if (args->num_seqs == 0) return LA_SUCCESS;
   info->attention = plan.mfma ? LA_PLAN_ATTENTION_MFMA : plan.f32 ? LA_PLAN_ATTENTION_MFMA_F32 : LA_PLAN_ATTENTION_VALU;
   info->chunk_rows = plan.chunk_len;

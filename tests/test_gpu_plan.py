@@ -76,3 +76,17 @@ def test_filled_pieces_stay_within_the_kernels_chunk_length(cuda, heads, num_seq
     if filled:
         n = i.num_chunks - num_seqs
         assert (num_seqs * seq_len + n - 1) // n <= 1 << 20
+
+
+@pytest.mark.parametrize("heads,seq_len", [(1, 100000), (3, 50000), (16, 100000), (128, 1000)])
+def test_float32_workspace_serves_any_alignment(cuda, heads, seq_len):
+    """Alignment decides which float32 kernel runs; a workspace sized with one set of pointers holds
+    the step over any other."""
+    size = lambda **kw: capi.load().la_mla_decode_workspace_size(ctypes.byref(plan_args("f32", heads, 1, seq_len, **kw)))
+    valu, mfma = size(kernel_variant=1), size()
+    assert plan("f32", heads, 1, seq_len).attention == F32
+    assert valu <= mfma
+    for name in ("kv_cache", "q_rope", "rope_cos", "rope_sin", "workspace"):
+        kw = {name: 0x10004}
+        assert plan("f32", heads, 1, seq_len, **kw).attention == VALU
+        assert size(**kw) == mfma == plan("f32", heads, 1, seq_len, **kw).workspace_bytes
