@@ -6,7 +6,8 @@ their phase boundaries; the shipped library has none of them). This script
 loads that build, runs decode steps of the benchmark workloads on cuda:0 and
 prints, per workload:
 
-* the attention kernel (``decode_mfma_kernel``): shader-clock cycles per wave
+* the attention kernel (``decode_mfma_kernel``; a workload that runs
+  ``decode_mfma16_kernel`` has no such table): shader-clock cycles per wave
   of each phase, mean and max over the waves of all workgroups, for two
   launches: the 10th of 10 identical launches back to back, and the launch
   inside a normal step (after the absorb kernel); and the mean cycles per
@@ -84,6 +85,11 @@ def load_phase_lib():
 SLOTS = 16  # kStampSlots in la_mfma.hip
 
 
+def attention_workgroups(info, heads: int) -> int:
+    """Workgroups of the attention launch of a plan over `heads` query heads per sequence."""
+    return 8 * -(-info.num_chunks * -(-heads // info.heads_per_workgroup) // 8)
+
+
 def attn_table(lib, blocks: int):
     import numpy as np
 
@@ -91,6 +97,8 @@ def attn_table(lib, blocks: int):
     assert lib.la_phase_attn_stamps(buf, blocks, 0) == 0
     full = np.frombuffer(buf, dtype=np.uint64).reshape(blocks, 4, SLOTS).astype(np.int64)
     full = full[full[:, 0, 10] > 0]  # workgroups that ran to the end
+    if len(full) == 0:
+        return None  # another attention kernel ran (decode_mfma16_kernel records no stamps)
     a = full[:, :, :11]
     d = np.diff(a, axis=2)
     total = a[:, :, 10] - a[:, :, 0]
@@ -107,6 +115,22 @@ def side_table(lib, kind: int, blocks: int):
     a = np.frombuffer(buf, dtype=np.uint64).reshape(blocks, 8).astype(np.int64)[:, :6]
     a = a[a[:, 5] > 0]
     return a
+
+
+def print_attention(rows) -> None:
+    print("\n| phase (cycles per wave) | back to back: mean | max | in a step: mean | max |")
+    print("|---|---|---|---|---|")
+    for i, ph in enumerate(ATTN_PHASES):
+        b, s = rows["back to back"][2][:, :, i], rows["in a step"][2][:, :, i]
+        print(f"| {ph} | {b.mean():.0f} | {b.max():.0f} | {s.mean():.0f} | {s.max():.0f} |")
+    tb, ts = rows["back to back"][1], rows["in a step"][1]
+    print(f"| total | {tb.mean():.0f} | {tb.max():.0f} | {ts.mean():.0f} | {ts.max():.0f} |")
+    print("\n| loop iteration part (cycles per tile, mean over waves) | back to back | in a step |")
+    print("|---|---|---|")
+    pb, ps = rows["back to back"][3], rows["in a step"][3]
+    for i, part in enumerate(TILE_PARTS):
+        print(f"| {part} | {pb[:, :, i].mean():.0f} | {ps[:, :, i].mean():.0f} |")
+    print(f"| iteration | {pb.sum(axis=2).mean():.0f} | {ps.sum(axis=2).mean():.0f} |")
 
 
 def pct(x, q):
@@ -147,7 +171,7 @@ def main() -> None:
         step = bench.Stepper(lib, capi, inp, stream)
         info = capi.PlanInfo()
         assert lib.la_mla_decode_plan(ctypes.byref(step.a), ctypes.byref(info)) == capi.LA_SUCCESS
-        ablocks = 8 * ((info.num_chunks * info.head_groups + 7) // 8)
+        ablocks = attention_workgroups(info, step.a.queries_per_seq * step.a.cfg.num_heads)
         for _ in range(30):
             step()
         bench.settle_clocks(step, 100)
@@ -165,19 +189,10 @@ def main() -> None:
         torch.cuda.synchronize()
         rows["in a step"] = attn_table(lib, ablocks)
         print(f"\nattention kernel (instrumented), back to back: {np.median(kern) * 1e3:.2f} us per launch", flush=True)
-        print("\n| phase (cycles per wave) | back to back: mean | max | in a step: mean | max |")
-        print("|---|---|---|---|---|")
-        for i, ph in enumerate(ATTN_PHASES):
-            b, s = rows["back to back"][2][:, :, i], rows["in a step"][2][:, :, i]
-            print(f"| {ph} | {b.mean():.0f} | {b.max():.0f} | {s.mean():.0f} | {s.max():.0f} |")
-        tb, ts = rows["back to back"][1], rows["in a step"][1]
-        print(f"| total | {tb.mean():.0f} | {tb.max():.0f} | {ts.mean():.0f} | {ts.max():.0f} |")
-        print("\n| loop iteration part (cycles per tile, mean over waves) | back to back | in a step |")
-        print("|---|---|---|")
-        pb, ps = rows["back to back"][3], rows["in a step"][3]
-        for i, part in enumerate(TILE_PARTS):
-            print(f"| {part} | {pb[:, :, i].mean():.0f} | {ps[:, :, i].mean():.0f} |")
-        print(f"| iteration | {pb.sum(axis=2).mean():.0f} | {ps.sum(axis=2).mean():.0f} |")
+        if rows["in a step"] is None:
+            print(f"\n(workgroups of {info.heads_per_workgroup} heads: decode_mfma16_kernel, which has no phase stamps)")
+        else:
+            print_attention(rows)
         # absorb and merge of that step
         for kind, kname, phases in ((0, "absorb", ABSORB_PHASES), (1, "merge + projection", MERGE_PHASES)):
             a = side_table(lib, kind, 8192)
