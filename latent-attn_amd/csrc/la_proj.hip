@@ -644,8 +644,9 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_kernel(DecodeProb
 
 // Merge + W_UV projection over one latent half, for launches with fewer
 // (head, row block) workgroups than CUs (a few query rows): one workgroup of
-// 8 waves per (head h, rpb <= 8 query rows, latent half c) merges the half rows
-// (fp16 slots, 512 B each) and multiplies them by W_UV's columns 256 c ..
+// 8 waves per (head h, rpb query rows, latent half c) merges the half rows
+// (fp16 slots, 512 B each; up to 8 rows, each over 8 / rows waves, or, with
+// kTasks = 2, up to 16, two per wave) and multiplies them by W_UV's columns 256 c ..
 // 256 c + 255 (64 KB per head), so twice as many workgroups move half the
 // bytes each. Both halves add their products into out with float atomics;
 // the kernel that writes the attention kernel's 16-bit queries
@@ -655,7 +656,7 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_kernel(DecodeProb
 constexpr int kMPHPitch = 256 + 8;  // 16-bit elements per LDS operand row (528 B: 16 B past 2 x 256)
 constexpr int kMPHSum = 256 + 4;    // floats per LDS row of a slot-group sum
 
-template <typename WT, int NB>
+template <typename WT, int NB, int kTasks>
 __global__ __launch_bounds__(kMPWaves * 64) void merge_project_half_kernel(DecodeProblem p, int rpb_log2) {
   LA_RSTAMP_DECL;
   LA_RSTAMP(0);
@@ -701,23 +702,32 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_half_kernel(Decod
     *reinterpret_cast<vec4*>(&oh[r * kMPHPitch + c0]) = hi;
     *reinterpret_cast<vec4*>(&ol[r * kMPHPitch + c0]) = lo;
   };
-  // each row's slots over G = 8 / rows waves (rows <= 8)
-  const int G = kMPWaves / rows;
-  const int r = wave / G, g = wave % G;
-  const int t[1] = {r < rows ? rb * rpb + r : -1};
-  f32x4 o[1][2];
-  merge_tasks<true, true, NB, 1>(p, t, h, g, G, lane, o, c);
-  LA_RSTAMP(2);
-  *reinterpret_cast<f32x4*>(&gp[wave * kMPHSum + 4 * lane]) = o[0][0];
-  __syncthreads();
-  // O half row r = sum of the G group rows of waves r G .. r G + G - 1; the
-  // block's other rows are zero
-  for (int i = tid; i < kMPRows * 64; i += kMPWaves * 64) {
-    const int rr = i / 64, c4 = i % 64;
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (rr < rows)
-      for (int q = 0; q < G; ++q) v += *reinterpret_cast<const f32x4*>(&gp[(rr * G + q) * kMPHSum + 4 * c4]);
-    put4(rr, 4 * c4, v);
+  if (kTasks == 2 && rows > kMPWaves) {
+    const int t[2] = {rb * rpb + wave, wave + kMPWaves < rows ? rb * rpb + wave + kMPWaves : -1};
+    f32x4 o[2][2];
+    merge_tasks<true, true, NB, 2>(p, t, h, 0, 1, lane, o, c);
+    LA_RSTAMP(2);
+    put4(wave, 4 * lane, o[0][0]);
+    put4(wave + kMPWaves, 4 * lane, o[1][0]);  // 0 without a second row
+  } else {
+    // each row's slots over G = 8 / rows waves
+    const int G = kMPWaves / rows;
+    const int r = wave / G, g = wave % G;
+    const int t[1] = {r < rows ? rb * rpb + r : -1};
+    f32x4 o[1][2];
+    merge_tasks<true, true, NB, 1>(p, t, h, g, G, lane, o, c);
+    LA_RSTAMP(2);
+    *reinterpret_cast<f32x4*>(&gp[wave * kMPHSum + 4 * lane]) = o[0][0];
+    __syncthreads();
+    // O half row r = sum of the G group rows of waves r G .. r G + G - 1; the
+    // block's other rows are zero
+    for (int i = tid; i < kMPRows * 64; i += kMPWaves * 64) {
+      const int rr = i / 64, c4 = i % 64;
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+      if (rr < rows)
+        for (int q = 0; q < G; ++q) v += *reinterpret_cast<const f32x4*>(&gp[(rr * G + q) * kMPHSum + 4 * c4]);
+      put4(rr, 4 * c4, v);
+    }
   }
   __syncthreads();
 
@@ -896,29 +906,35 @@ hipError_t launch_combine_project_mfma(const DecodeProblem& p, hipStream_t strea
   if (halves) {
     if (!p.part_f16) return hipErrorInvalidValue;
     // id = 8 (2 (head / 8 * nrb + row block) + half) + head % 8
-    // Rows per workgroup: 8, one per wave (with 16, two: 16 rows x 16 slots x
-    // 128 heads took 16.0 us against 13.6), halved while the launch leaves CUs
-    // idle (32 rows x 17 slots x 16 heads: 9.9 us with 8 rows, 64 CUs; 7.5 with
-    // 4; 9.0 with 2, where workgroups pay their fixed part twice per CU).
-    const int hb = 2 * 8 * ((p.nh + 7) / 8);
-    int rpb_log2 = 3;
-    while (rpb_log2 > 0 && hb * ((R + (1 << rpb_log2) - 1) >> rpb_log2) < ncu) --rpb_log2;
-    const int rpb = 1 << rpb_log2;
-    const dim3 grid((unsigned)(hb * ((R + rpb - 1) >> rpb_log2)));
     // Slots per row: seq_len / chunk_len with equal sequences whose chunks align
     // with them, else up to two more; a sequence's share of the chunks where
-    // the lengths are on the device. The rows of a block share G = 8 / rows
-    // tasks, which load 8, 16 or 32 slots at once (kMPSlots).
-    const int G = kMPWaves / (R < rpb ? R : rpb);
+    // the lengths are on the device.
     const int64_t n = p.offsets || p.lens || p.chunk_len <= 0 ? p.num_chunks / p.num_seqs
                       : p.seq_len % p.chunk_len == 0          ? p.seq_len / p.chunk_len
                                                               : p.seq_len / p.chunk_len + 2;
+    // Rows per workgroup: 8, one per wave, or 16, two per wave, where all slots
+    // of two rows go out at once (kMPSlots): the W_UV rows are then read by half
+    // as many workgroups. us with 16 and with 8 rows: 64 rows x 5 slots x 48
+    // heads 12.3 / 14.7, 128 x 8 x 16 heads 10.1 / 11.2, 12 x 8 x 128 heads 9.6 /
+    // 10.8; with 16 slots, two batches, 16 rows x 128 heads 15.5 / 14.1. Halved
+    // while the launch leaves CUs idle (32 rows x 17 slots x 16 heads: 10.9 us
+    // with 8 rows, 64 CUs; 7.6 with 4; 9.1 with 2, where workgroups pay their
+    // fixed part twice per CU).
+    const int hb = 2 * 8 * ((p.nh + 7) / 8);
+    int rpb_log2 = n <= kMPSlots && R > kMPWaves ? 4 : 3;
+    while (rpb_log2 > 0 && hb * ((R + (1 << rpb_log2) - 1) >> rpb_log2) < ncu) --rpb_log2;
+    const int rpb = 1 << rpb_log2;
+    const dim3 grid((unsigned)(hb * ((R + rpb - 1) >> rpb_log2)));
+    // The rows of a block share G = 8 / rows tasks, which load 8, 16 or 32 slots
+    // at once (kMPSlots).
+    const int G = rpb > kMPWaves ? 1 : kMPWaves / (R < rpb ? R : rpb);
     const int64_t per = (n + G - 1) / G;
     const bool bf = p.wuv_dtype == LA_DTYPE_BF16;
-    auto k = per > 16 ? (bf ? merge_project_half_kernel<__hip_bfloat16, 32> : merge_project_half_kernel<__half, 32>)
-             : per > kMPSlots ? (bf ? merge_project_half_kernel<__hip_bfloat16, 16> : merge_project_half_kernel<__half, 16>)
-                              : (bf ? merge_project_half_kernel<__hip_bfloat16, kMPSlots>
-                                    : merge_project_half_kernel<__half, kMPSlots>);
+    typedef __hip_bfloat16 B;
+    auto k = rpb > kMPWaves   ? (bf ? merge_project_half_kernel<B, kMPSlots, 2> : merge_project_half_kernel<__half, kMPSlots, 2>)
+             : per > 16       ? (bf ? merge_project_half_kernel<B, 32, 1> : merge_project_half_kernel<__half, 32, 1>)
+             : per > kMPSlots ? (bf ? merge_project_half_kernel<B, 16, 1> : merge_project_half_kernel<__half, 16, 1>)
+                              : (bf ? merge_project_half_kernel<B, kMPSlots, 1> : merge_project_half_kernel<__half, kMPSlots, 1>);
     hipLaunchKernelGGL(k, grid, dim3(kMPWaves * 64), 0, stream, p, rpb_log2);
     return hipGetLastError();
   }
