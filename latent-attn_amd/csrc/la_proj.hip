@@ -524,10 +524,8 @@ __device__ inline void merge_tasks(const DecodeProblem& p, const int (&t)[kTasks
 constexpr int kMPWaves = 8;
 // slot rows each task loads up front (one memory round trip for up to this
 // many; more loop over further batches, a round trip each). The half-row merge
-// also comes with 16 and 32 (8 B per lane each), taken by the slots per task:
-// 8 / 16 / 32 at once take 14.5 / 13.9 / 18.7 us for 16 slots, 18.9 / 19.6 /
-// 15.6 for 32, 5.9 / 6.0 / 6.4 for one (88, 104 and 136 VGPRs: fewer
-// workgroups per CU).
+// also comes with 16 and 32 (8 B per lane each; 88, 104 and 136 VGPRs with one
+// row per wave, 108, 140 and 205 with two), taken by the launch's rule.
 constexpr int kMPSlots = 8;
 constexpr int kMPPitch = kDcP + 4;  // floats per LDS row of a slot-group sum
 // 16-bit elements per LDS row of the high / low operand rows: 1040 B, 16 B
@@ -912,29 +910,44 @@ hipError_t launch_combine_project_mfma(const DecodeProblem& p, hipStream_t strea
     const int64_t n = p.offsets || p.lens || p.chunk_len <= 0 ? p.num_chunks / p.num_seqs
                       : p.seq_len % p.chunk_len == 0          ? p.seq_len / p.chunk_len
                                                               : p.seq_len / p.chunk_len + 2;
-    // Rows per workgroup: 8, one per wave, or 16, two per wave, where all slots
-    // of two rows go out at once (kMPSlots): the W_UV rows are then read by half
-    // as many workgroups. us with 16 and with 8 rows: 64 rows x 5 slots x 48
-    // heads 12.3 / 14.7, 128 x 8 x 16 heads 10.1 / 11.2, 12 x 8 x 128 heads 9.6 /
-    // 10.8; with 16 slots, two batches, 16 rows x 128 heads 15.5 / 14.1. Halved
-    // while the launch leaves CUs idle (32 rows x 17 slots x 16 heads: 10.9 us
-    // with 8 rows, 64 CUs; 7.6 with 4; 9.1 with 2, where workgroups pay their
-    // fixed part twice per CU).
+    // Rows per workgroup: 8, one per wave, or 16, two per wave, so that half as
+    // many workgroups read the W_UV rows; both halved while the launch leaves CUs
+    // idle. 16 where all slots of two rows go out at once (kMPSlots; us with 16
+    // and with 8 rows: 64 rows x 5 slots x 48 heads 12.3 / 14.7, 128 x 8 x 16
+    // heads 10.1 / 11.2, 12 x 8 x 128 heads 9.6 / 10.8), and where they take one
+    // workgroup per CU at most and the last block of a head has room for four
+    // more rows, so that 8 rows would be about as many tasks per CU and twice the
+    // weights (128 heads: 10 rows x 16 / 25 slots 11.6 / 15.0 against 12.7 / 16.9,
+    // 12 rows 12.3 / 16.1 against 13.1 / 17.9; 14 rows 14.3 / 18.7 against 13.6 /
+    // 18.2, 16 rows 15.0 / 19.5 against 14.4 / 18.8). 4 or fewer: 32 rows x 17
+    // slots x 16 heads take 10.9 us with 8 rows, 64 CUs; 7.6 with 4; 9.1 with 2,
+    // where workgroups pay their fixed part twice per CU.
     const int hb = 2 * 8 * ((p.nh + 7) / 8);
-    int rpb_log2 = n <= kMPSlots && R > kMPWaves ? 4 : 3;
-    while (rpb_log2 > 0 && hb * ((R + (1 << rpb_log2) - 1) >> rpb_log2) < ncu) --rpb_log2;
+    const int blocks16 = hb * nrb, room = kMPRows * nrb - R;
+    const bool two = R > kMPWaves && 4 * blocks16 >= 3 * ncu && (n <= kMPSlots || (blocks16 <= ncu && room >= 4));
+    int rpb_log2 = two ? 4 : 3;
+    while (!two && rpb_log2 > 0 && hb * ((R + (1 << rpb_log2) - 1) >> rpb_log2) < ncu) --rpb_log2;
     const int rpb = 1 << rpb_log2;
     const dim3 grid((unsigned)(hb * ((R + rpb - 1) >> rpb_log2)));
-    // The rows of a block share G = 8 / rows tasks, which load 8, 16 or 32 slots
-    // at once (kMPSlots).
-    const int G = rpb > kMPWaves ? 1 : kMPWaves / (R < rpb ? R : rpb);
+    // Up to 8 rows of a block share G = 8 / rows tasks each. A task loads 8, 16 or
+    // 32 slots at once; 32 (136 VGPRs with one row per wave: one workgroup per CU)
+    // only where no CU has a second workgroup, with two the launch takes two
+    // rounds (us with 16 and with 32 slots at once: 16 rows x 17 / 24 / 32 slots x
+    // 128 heads, 512 workgroups, 15.4 / 18.0 / 21.1 and 19.2 / 21.6 / 24.7; 8 rows x
+    // 32 slots, 256 workgroups, 16.4 and 14.2).
+    const int G = two ? 1 : kMPWaves / (R < rpb ? R : rpb);
     const int64_t per = (n + G - 1) / G;
-    const bool bf = p.wuv_dtype == LA_DTYPE_BF16;
+    const int batch = per <= kMPSlots ? 0 : per <= 16 || (int)grid.x > ncu ? 1 : 2;
+    typedef void (*Kernel)(DecodeProblem, int);
     typedef __hip_bfloat16 B;
-    auto k = rpb > kMPWaves   ? (bf ? merge_project_half_kernel<B, kMPSlots, 2> : merge_project_half_kernel<__half, kMPSlots, 2>)
-             : per > 16       ? (bf ? merge_project_half_kernel<B, 32, 1> : merge_project_half_kernel<__half, 32, 1>)
-             : per > kMPSlots ? (bf ? merge_project_half_kernel<B, 16, 1> : merge_project_half_kernel<__half, 16, 1>)
-                              : (bf ? merge_project_half_kernel<B, kMPSlots, 1> : merge_project_half_kernel<__half, kMPSlots, 1>);
+    static const Kernel bf16[2][3] = {
+        {merge_project_half_kernel<B, kMPSlots, 1>, merge_project_half_kernel<B, 16, 1>, merge_project_half_kernel<B, 32, 1>},
+        {merge_project_half_kernel<B, kMPSlots, 2>, merge_project_half_kernel<B, 16, 2>, merge_project_half_kernel<B, 32, 2>}};
+    typedef __half H;
+    static const Kernel f16[2][3] = {
+        {merge_project_half_kernel<H, kMPSlots, 1>, merge_project_half_kernel<H, 16, 1>, merge_project_half_kernel<H, 32, 1>},
+        {merge_project_half_kernel<H, kMPSlots, 2>, merge_project_half_kernel<H, 16, 2>, merge_project_half_kernel<H, 32, 2>}};
+    const Kernel k = (p.wuv_dtype == LA_DTYPE_BF16 ? bf16 : f16)[two][batch];
     hipLaunchKernelGGL(k, grid, dim3(kMPWaves * 64), 0, stream, p, rpb_log2);
     return hipGetLastError();
   }

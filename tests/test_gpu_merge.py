@@ -24,6 +24,8 @@ pytestmark = pytest.mark.gpu
     (128, 8, 256, 32), (128, 9, 256, 32), (128, 12, 70, 32), (128, 15, 250, 64), (128, 16, 256, 32),  # 16 rows, <= 8 slots
     (48, 17, 96, 32), (48, 64, 160, 64), (16, 130, 96, 32),  # with a last block of 1, 16 and 2 rows
     (128, 9, 288, 32), (128, 16, 512, 32), (128, 16, 544, 32), (128, 3, 1000, 16),  # more slots: 8 rows, or waves per row
+    (128, 8, 544, 32), (128, 16, 1056, 32),  # one and two workgroups per CU: batches of 32 and of 16
+    (128, 9, 1056, 32), (128, 12, 288, 32), (128, 13, 544, 32), (48, 24, 850, 50),  # room for seven, four, three rows
 ])
 def test_rows_and_slots(cuda, dtype, heads, B, S, chunk):
     if torch.cuda.get_device_properties(cuda).multi_processor_count == 256:
