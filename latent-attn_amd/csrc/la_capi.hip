@@ -176,9 +176,13 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
     min_rows = std::min<int64_t>(L, 128);
   } else if (few_heads && !coarse) {
     // two workgroups per CU and no more (16 heads x 131168 rows: 33.4 us with
-    // 257-row chunks, 37 with 128, 35.6 with 513); whole tiles only where a
-    // paged cache needs them, so that rounding leaves no CU without a chunk
-    const int64_t chunks = std::max<int64_t>(1, 2LL * ncu / heads16);
+    // 257-row chunks, 37 with 128, 35.6 with 513), but one while a sequence has
+    // more than 128 chunks: its row's merge reads them all in a few workgroups
+    // (16 heads, a step over 1 x 32768 rows 41.4 us with 512 chunks, 29.1 with
+    // 256; 1 x 131072 60.6 and 48.1; 3 x 30000 40.7 and, with 384, 37.6; 4 x 32768
+    // 45.5 and 43.5; 32 x 4099 46.5 and 49.2); whole tiles only where a paged cache
+    // needs them, so that rounding leaves no CU without a chunk
+    const int64_t chunks = std::max<int64_t>(std::min(2LL * ncu / heads16, 128LL * a->num_seqs), ncu);
     L = (total + chunks - 1) / chunks;
     L = std::max<int64_t>((L + 15) / 16 * 16, 64);
   } else {

@@ -90,3 +90,19 @@ def test_float32_workspace_serves_any_alignment(cuda, heads, seq_len):
         kw = {name: 0x10004}
         assert plan("f32", heads, 1, seq_len, **kw).attention == VALU
         assert size(**kw) == mfma == plan("f32", heads, 1, seq_len, **kw).workspace_bytes
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp8"])
+@pytest.mark.parametrize("num_seqs,seq_len,heads,want", [
+    (1, 8192, 16, 128), (1, 32768, 16, 256), (1, 131072, 16, 256), (2, 32768, 16, 256), (3, 32768, 16, 384),
+    (4, 32768, 16, 512), (32, 4099, 16, 483), (1, 32768, 32, 256),
+])
+def test_few_heads_keep_the_slots_of_a_sequence_few(cuda, dtype, num_seqs, seq_len, heads, want):
+    """Two chunks per CU at 16 heads, but no more than 128 per sequence while one per CU remains: the
+    merge of a query row reads a slot per chunk in a few workgroups."""
+    import torch
+
+    if torch.cuda.get_device_properties(cuda).multi_processor_count != 256:
+        pytest.skip("the counts are of 256 CUs")
+    i = plan(dtype, heads, num_seqs, seq_len)
+    assert (i.num_chunks, i.heads_per_workgroup) == (want, 16)
