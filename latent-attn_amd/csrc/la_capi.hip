@@ -155,12 +155,23 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
 
   const int64_t total = paged ? p->total_rows : a->seq_offsets ? a->total_rows : (int64_t)a->num_seqs * a->seq_len;
   const int ncu = cu_count();
-  // Up to 32 query heads always take the 16-head kernel: 128-head workgroups
-  // run the matrix work of 128 heads whatever their number (32 x 4099 rows,
-  // attention us, 128-head against 16-head workgroups: 16 heads 51 / 33, 32
-  // heads 52 / 38, 64 heads 53 / 60).
+  // Up to 32 query heads take the 16-head kernel: 128-head workgroups run the
+  // matrix work of 128 heads whatever their number (32 x 4099 rows, attention us,
+  // 128-head against 16-head workgroups: 16 heads 51 / 33, 32 heads 52 / 38, 64
+  // heads 53 / 60). With 17 to 32, two workgroups read each row, and once a
+  // 16-bit cache streams from HBM (not from the 256 MB behind the L2s) their
+  // shorter tiles in flight fall behind (a step over one sequence: 196,608 rows
+  // 78.2 / 76.5, 212,992 81.0 / 86.3, 262,144 93.7 / 105.0; 32 sequences of 163,840
+  // in all 66.2 / 51.2, 245,760 89.0 / 86.0, 262,144 92.8 / 93.4; 64 over 327,680
+  // 112.8 / 115.1). FP8 rows stay (64 x 8192: 155 / 126), and so do caches cut
+  // over their filled rows, whose number only the device knows (64 regions of
+  // 8192 rows, a step with 128-head workgroups over the regions and this one:
+  // full 164 / 169, three quarters 147 / 152, half 123 / 98, a quarter 118 / 55).
   const int heads16 = pl.mfma ? p->Hq / 16 : 0;
-  const bool few_heads = pl.mfma && heads16 <= 2;
+  const bool by_fill = a->seq_lens && chunk_rows == 0 && 4LL * a->num_seqs <= ncu;
+  const int64_t most16 = a->num_seqs == 1 ? 200000 : 240000;
+  const bool few_heads = pl.mfma && (heads16 == 1 || (heads16 == 2 && (a->kv_dtype == LA_DTYPE_FP8_E4M3 || by_fill ||
+                                                                       total <= most16)));
   int64_t L, min_rows = 64;
   if (chunk_rows > 0) {
     L = chunk_rows;
@@ -221,7 +232,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
   // 128 heads 16.2 us on the 128-head kernel, 7.9 here; 1 x 8192 17.0 / 11.6;
   // four times that (16 queries over 2048 rows) 21.7 / 36.3. With at most one
   // workgroup per CU, 8 waves take 128 positions per round trip.
-  if (pl.mfma && (few_heads || nchunks * heads16 <= 2 * ncu))
+  if (pl.mfma && (few_heads || (heads16 > 2 && nchunks * heads16 <= 2 * ncu)))
     pl.waves16 = nchunks * heads16 <= ncu && L >= 128 ? 8 : 4;
   pl.num_slots = nchunks > 0 ? (int)(nchunks + a->num_seqs - 1) : 0;
 

@@ -1,7 +1,8 @@
 """The 16-head MFMA attention kernel (csrc/la_mfma16.hip) at the edges of its
 tiles (16 rows per wave, 64 or 128 positions), over every cache layout and
-type it serves, against the float64 oracle. Up to 32 query heads always take
-it; 128 heads do while its workgroups fill the chip at most twice."""
+type it serves, against the float64 oracle. Up to 32 query heads take it (32
+over 16-bit caches within the infinity cache); more do while its workgroups
+fill the chip at most twice."""
 
 from __future__ import annotations
 

@@ -106,3 +106,17 @@ def test_few_heads_keep_the_slots_of_a_sequence_few(cuda, dtype, num_seqs, seq_l
         pytest.skip("the counts are of 256 CUs")
     i = plan(dtype, heads, num_seqs, seq_len)
     assert (i.num_chunks, i.heads_per_workgroup) == (want, 16)
+
+
+@pytest.mark.parametrize("dtype,heads,num_seqs,seq_len,want", [
+    ("bf16", 16, 64, 8192, 16), ("bf16", 32, 32, 4099, 16), ("f16", 32, 30, 8000, 16), ("f16", 32, 30, 8001, 128),
+    ("bf16", 32, 1, 200000, 16), ("bf16", 32, 1, 200001, 128), ("fp8", 32, 64, 8192, 16),
+    ("bf16", 48, 1, 8192, 16), ("bf16", 48, 32, 4099, 128),
+])
+def test_few_heads_over_large_caches(cuda, dtype, heads, num_seqs, seq_len, want):
+    """32 heads leave the 16-head kernel where their 16-bit cache outgrows the infinity cache."""
+    i = plan(dtype, heads, num_seqs, seq_len)
+    assert i.attention == MFMA and i.heads_per_workgroup == want
+    if heads == 32:  # with lengths only the device knows how many rows stream
+        assert plan(dtype, heads, num_seqs, seq_len, **LENS).heads_per_workgroup == 16
+        assert plan(dtype, heads, num_seqs, seq_len, chunk_rows=512, **LENS).heads_per_workgroup == want
