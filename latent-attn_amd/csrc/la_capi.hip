@@ -263,7 +263,7 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
   pl.part_lse_off = off;
   const int piece = (int)std::min<int64_t>((min_rows + 31) / 32 * 32, L);  // shortest piece of filled rows
   const bool filled = a->seq_lens && chunk_rows == 0 && (pl.mfma || pl.f32) && 4LL * a->num_seqs <= nchunks &&
-                      total <= INT32_MAX &&
+                      total <= INT32_MAX && (L > piece || a->seq_offsets || p->seq_len % L != 0) &&
                       piece_rows((uint32_t)total, (uint32_t)(nchunks - a->num_seqs), piece) <= kMaxChunkRows;
   off += align_up((size_t)pl.num_slots * p->Hq * sizeof(float));
   pl.proj_mfma = project_mfma_supported(*p);
@@ -276,7 +276,10 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
   // more per sequence (100 sequences of 100 to 4000 rows over 256 chunks, too
   // uneven pieces: 165 us a step against 147 over their 4096-row regions; 64 of
   // 300 to 8192: 120 against 154; 32 of 500 to 8000 in 32768-row regions: 74
-  // against 208).
+  // against 208), and unless the regions' chunks are already of that length and
+  // end with their regions: the pieces would be the same ones, found again on
+  // the device (32 of 100 to 500 rows in 512-row regions, 128 heads: 36.4 against
+  // 35.5, fp8 38.5 against 37.1).
   if (filled) p->chunk_len = -piece;
   p->num_chunks = pl.num_chunks;
   p->num_slots = pl.num_slots;

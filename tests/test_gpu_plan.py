@@ -120,3 +120,19 @@ def test_few_heads_over_large_caches(cuda, dtype, heads, num_seqs, seq_len, want
     if heads == 32:  # with lengths only the device knows how many rows stream
         assert plan(dtype, heads, num_seqs, seq_len, **LENS).heads_per_workgroup == 16
         assert plan(dtype, heads, num_seqs, seq_len, chunk_rows=512, **LENS).heads_per_workgroup == want
+
+
+@pytest.mark.parametrize("heads,num_seqs,seq_len,kw,filled", [
+    (128, 32, 512, {}, 0),                          # chunks of 128 rows end with the regions: the pieces are the same
+    (128, 32, 512, {"seq_offsets": 0x10000}, 1),    # regions of any length
+    (128, 32, 520, {}, 1),                          # chunks across regions
+    (128, 16, 8192, {}, 1),                         # 512-row chunks, pieces down to 128
+    (16, 32, 1024, {}, 0), (16, 32, 2048, {}, 1),   # 64-row and 128-row chunks of the 16-head kernel
+])
+def test_filled_rows_are_cut_where_that_makes_other_pieces(cuda, heads, num_seqs, seq_len, kw, filled):
+    import torch
+
+    if torch.cuda.get_device_properties(cuda).multi_processor_count != 256:
+        pytest.skip("the sizes are of 256 CUs")
+    i = plan("bf16", heads, num_seqs, seq_len, **LENS, **kw)
+    assert i.num_chunks >= 4 * num_seqs and i.filled_rows == filled
