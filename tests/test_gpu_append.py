@@ -229,3 +229,23 @@ def test_append_prompt(cuda, cache_dtype, src_dtype, bs, shift, tokens):
     got = q_dev.cpu().numpy().astype(np.float64)
     assert np.all(np.abs(got - rot)[:2 * qps] <= 1e-5 + 1e-5 * np.abs(rot)[:2 * qps])
     assert torch.equal(q_dev[2 * qps:].cpu(), q[2 * qps:])
+
+
+# both sides of the limit of one element per thread (1,024 elements, 2,560 into an FP8 cache)
+@pytest.mark.parametrize("src_dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("tokens", [1, 2, 4, 5])
+def test_fp8_append_of_a_few_tokens(cuda, src_dtype, tokens):
+    cfg = MLAConfig.deepseek_v2()
+    B, cap = 3, 16
+    kv = torch.zeros(B, cap, ROW, dtype=torch.float8_e4m3fn, device=cuda)
+    lens0 = [0, 3, cap - tokens]
+    lens = torch.tensor(lens0, dtype=torch.int32, device=cuda)
+    c_t, k_rope = new_rows(B, tokens, src_dtype, 71)
+    F.append_kv(kv, lens, c_t.to(cuda), k_rope.to(cuda), cfg)
+    torch.cuda.synchronize()
+    want = mo.fp8_e4m3_encode(np.concatenate([to_np(c_t), to_np(k_rope)], axis=-1))
+    codes = kv.view(torch.uint8).cpu().numpy()
+    for b, n in enumerate(lens0):
+        assert np.array_equal(codes[b, n:n + tokens], want[b])
+        assert not codes[b, :n].any() and not codes[b, n + tokens:].any()
+    assert lens.cpu().tolist() == [n + tokens for n in lens0]
