@@ -70,6 +70,8 @@ struct DecodeProblem {
   int qps;                // query tokens per sequence
   int nh;                 // weight heads
   int Hq;                 // query heads per sequence = qps * nh
+  int merge_rows_log2;    // half-row merge: log2 of its query rows per workgroup (in the padding before
+                          // the pointers, which one load brings with the three above)
   const float* q_abs;     // (num_seqs*Hq, dc) f32
   const float* q_rope;    // (num_seqs*Hq, dR) f32
   void* q_prep;           // MFMA path: [q_abs | q_rope] * scale_log2 in the MFMAs' 16-bit
@@ -110,6 +112,7 @@ struct DecodeProblem {
 __device__ inline void warm_kernarg_lines(const DecodeProblem& p) {
   asm volatile("" ::"s"(p.seq_len), "s"(p.Hq), "s"(p.rope_rows), "s"(p.num_chunks));
 }
+static_assert(offsetof(DecodeProblem, merge_rows_log2) == offsetof(DecodeProblem, qps) + 12, "one 16-B load");
 static_assert(offsetof(DecodeProblem, seq_len) < 64 && offsetof(DecodeProblem, Hq) / 64 == 1 &&
                   offsetof(DecodeProblem, rope_rows) / 64 == 2 && offsetof(DecodeProblem, num_chunks) / 64 == 3 &&
                   sizeof(DecodeProblem) + 4 <= 256,
