@@ -13,6 +13,9 @@ import torch
 from conftest import assert_close
 from mla_cases import cfg_with_heads, make_queries, make_weights, rope, staircase_case, to_np
 from oracle import mla_oracle as mo
+from test_gpu_plan import F32, VALU, plan
+
+from latent_attn import capi
 
 pytestmark = pytest.mark.gpu
 
@@ -29,6 +32,11 @@ def test_edges(cuda, layout, heads, chunk):
     cfg = cfg_with_heads(heads)
     lens = [1, 7, 8, 9, 31, 32, 33, 0, 63, 64, 65, 100, 5, 15, 16, 17, 40]  # 17 query rows: two merge blocks
     B, bs, per = len(lens), 32, 4
+    where = {"ragged": dict(seq_offsets=0x10000, total_rows=sum(lens)),
+             "paged": dict(seq_lens=0x10000, block_table=0x10000, block_size=bs, blocks_per_seq=per, total_rows=B * per * bs)}
+    i = plan("f32", heads, B, 0, chunk_rows=chunk, **where[layout])
+    assert (i.attention, i.heads_per_workgroup) == (F32, 16)
+    assert i.merge in (capi.LA_PLAN_MERGE_MFMA_F32, capi.LA_PLAN_MERGE_MFMA_F32_HALVES)
     W_UK, W_UV = make_weights(cfg, "f32", 3, cuda)
     q_nope, q_rope = make_queries((B,), cfg, 4, cuda)
     cos, sin = rope(max(lens), cfg, cuda)
@@ -112,8 +120,6 @@ def test_shared_cache_workspace(cuda, seq, heads):
 def test_absorb_into_an_output_that_is_only_float_aligned(cuda, shift):
     """The MFMA absorption stores 16-byte vectors: an output without that alignment takes the VALU
     kernel, as a q_nope without it does (the same bits)."""
-    from latent_attn import capi
-
     lib, cfg = capi.load(), cfg_with_heads(3)
     g = torch.Generator().manual_seed(11)
     q = torch.randn(5 * 3 * 128, generator=g).to(cuda)
@@ -142,9 +148,6 @@ def test_absorb_into_an_output_that_is_only_float_aligned(cuda, shift):
 @pytest.mark.parametrize("shift", [0, 4])
 def test_workspace_that_is_only_float_aligned(cuda, heads, shift):
     """A float32 step over a workspace without 16-byte alignment runs on the VALU kernels."""
-    from latent_attn import capi
-    from test_gpu_plan import F32, VALU
-
     lib, cfg = capi.load(), cfg_with_heads(heads)
     B, S = 2, 300
     W_UK, W_UV = make_weights(cfg, "f32", 3, cuda)

@@ -1,9 +1,10 @@
 """Decode with per-sequence lengths: the MFMA kernels' chunks share the filled
 rows, found on the device (seq_in_plan / ChunkWalk, csrc/la_internal.hpp).
 More sequences than a wave has lanes, empty ones, lengths around the padding
-of 32, one long sequence among short ones, over capacity, packed and paged
-caches, against the float64 oracle over the filled rows; unfilled rows hold
-values that would dominate any softmax."""
+of 32, one long sequence among short ones, pieces longer than the shortest,
+over capacity, packed and paged caches, against the float64 oracle over the
+filled rows; unfilled rows hold values that would dominate any softmax. The
+plan says that the pieces are of filled rows."""
 
 from __future__ import annotations
 
@@ -14,19 +15,32 @@ import torch
 from conftest import assert_close
 from mla_cases import TORCH_DTYPE, cfg_with_heads, make_queries, make_weights, rope, to_np
 from oracle import mla_oracle as mo
+from test_gpu_plan import plan
 
 pytestmark = pytest.mark.gpu
 
 
+SHORT = [0, 31, 32, 33, 0, 200, 64]  # a leading and a middle empty sequence
+MANY = [0, 31, 32, 33, 1, 0, 200] + [5, 64] * 33  # 73: more than a wave has lanes (at 128 heads never: 256 chunks)
+ALL = [("bf16", 128), ("fp8", 128), ("f16", 16), ("f32", 16)]
+CASES = [(lens, cap, dt, heads) for lens, cap, kinds in [
+    (SHORT, 544, ALL), (MANY, 544, ALL[2:]), ([0] * 3, 544, ALL), ([3000, 1, 40], 3040, ALL), ([2001], 3040, ALL),
+    ([10016, 9000, 10016, 9999], 10016, ALL[:3]),  # nearly full: pieces longer than the plan's shortest
+] for dt, heads in kinds]
+
+
 @pytest.mark.parametrize("layout", ["capacity", "packed", "paged"])
-@pytest.mark.parametrize("dtype,heads", [("bf16", 128), ("f16", 16), ("fp8", 128), ("f32", 16)])
-@pytest.mark.parametrize("lens", [[0, 31, 32, 33, 1, 0, 200] + [5, 64] * 33, [0] * 3, [3000, 1, 40], [2001]])
-def test_filled_rows(cuda, layout, dtype, heads, lens):
+@pytest.mark.parametrize("lens,cap,dtype,heads", CASES)
+def test_filled_rows(cuda, layout, dtype, heads, lens, cap):
     from latent_attn import functional as F
 
     cfg = cfg_with_heads(heads)
     B, bs = len(lens), 32
-    cap = 224 if max(lens) <= 200 else 3008
+    if torch.cuda.get_device_properties(cuda).multi_processor_count == 256:  # the sizes are of 256 CUs
+        i = plan(dtype, heads, B, 0 if layout == "paged" else cap, total_rows=B * cap, seq_lens=0x10000, **{
+            "capacity": {}, "packed": {"seq_offsets": 0x10000},
+            "paged": {"block_table": 0x10000, "block_size": bs, "blocks_per_seq": cap // bs}}[layout])
+        assert i.filled_rows == 1 and i.num_chunks >= 4 * B
     wt = {"fp8": "bf16"}.get(dtype, dtype)
     dt = torch.float8_e4m3fn if dtype == "fp8" else TORCH_DTYPE[dtype]
     W_UK, W_UV = make_weights(cfg, wt, 3, cuda)

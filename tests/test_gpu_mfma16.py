@@ -13,6 +13,7 @@ import torch
 from conftest import assert_close
 from mla_cases import TORCH_DTYPE, cfg_with_heads, make_queries, make_weights, rope, staircase_case, to_np
 from oracle import mla_oracle as mo
+from test_gpu_plan import MFMA, plan
 
 pytestmark = pytest.mark.gpu
 
@@ -35,6 +36,10 @@ def test_edges(cuda, layout, dtype, heads, chunk):
     cfg = cfg_with_heads(heads)
     lens = [1, 15, 16, 17, 63, 64, 65, 0, 127, 128, 129, 200]
     B, bs, per = len(lens), 32, 8
+    where = {"ragged": dict(seq_offsets=0x10000, total_rows=sum(lens)),
+             "paged": dict(seq_lens=0x10000, block_table=0x10000, block_size=bs, blocks_per_seq=per, total_rows=B * per * bs)}
+    i = plan(dtype, heads, B, 0, chunk_rows=chunk, kernel_variant=2, **where[layout])
+    assert (i.attention, i.heads_per_workgroup) == (MFMA, 16)
     wt = "f16" if dtype == "f16" else "bf16"
     W_UK, W_UV = make_weights(cfg, wt, 3, cuda)
     q_nope, q_rope = make_queries((B,), cfg, 4, cuda)
@@ -67,6 +72,7 @@ def test_rising_maximum(cuda, chunk):
     from latent_attn import functional as F
 
     cfg = cfg_with_heads(128)
+    assert plan("bf16", 128, 1, 700, chunk_rows=chunk, kernel_variant=2).heads_per_workgroup == 16
     kv, qa, qr = staircase_case(1, 700, "bf16", 6, cuda)
     _, W_UV = make_weights(cfg, "bf16", 7, cuda)
     cos, sin = rope(700, cfg, cuda)

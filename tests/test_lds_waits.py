@@ -4,7 +4,8 @@ register that an inline-asm LDS read (lgkmcnt) or vector-memory load
 vmcnt values, and the paged cache's block-table entries) has not yet written
 (see tests/lds_wait_check.py). Compiles latent-attn_amd/csrc/la_mfma.hip for
 gfx950 to assembly with hipcc (about half a minute) and checks every
-instantiation of decode_mfma_kernel. A compiler copy of such a register
+instantiation of decode_mfma_kernel and decode_mfma_filled_kernel (the same
+body with chunks over filled rows, allocated separately). A compiler copy of such a register
 before its wait once read a partner wave's rescale flag before it had landed;
 a count that released a wait early would show up the same way, as a use of a
 register whose load the in-order model has not retired. The kernels are
@@ -37,11 +38,22 @@ def decode_asm(tmp_path_factory):
     return out.read_text()
 
 
+# {bf16, f16, fp8} x {contiguous, paged}, and {bf16, f16, fp8} over the filled rows of contiguous caches
+KERNELS = {"_ZN2la12_GLOBAL__N_118decode_mfma_kernel": 6, "_ZN2la12_GLOBAL__N_125decode_mfma_filled_kernel": 3}
+
+
+def select(parse, asm):
+    out = {}
+    for prefix, count in KERNELS.items():
+        ks = parse(asm, prefix)
+        assert len(ks) == count, sorted(ks)
+        out.update(ks)
+    return out
+
+
 @pytest.fixture(scope="module")
 def decode_kernels(decode_asm):
-    ks = kernels(decode_asm, "_ZN2la12_GLOBAL__N_118decode_mfma_kernel")
-    assert len(ks) == 6, sorted(ks)  # {bf16, f16} x {contiguous, paged} and fp8 x {contiguous, paged}
-    return ks
+    return select(kernels, decode_asm)
 
 
 def test_checker_catches_an_early_copy():
@@ -120,8 +132,7 @@ def test_cfg_walk_skips_only_the_no_lane_outcome_of_a_divergent_if():
 
 
 def test_no_register_touched_before_its_wait_on_any_path(decode_asm):
-    ks = kernels_with_labels(decode_asm, "_ZN2la12_GLOBAL__N_118decode_mfma_kernel")
-    assert len(ks) == 6, sorted(ks)
+    ks = select(kernels_with_labels, decode_asm)
     for name, lines in ks.items():
         bad = pending_uses_cfg(lines, counters=("lgkm", "vm"))
         assert not bad, f"{name}: " + "; ".join(f"#{n} {ins!r} before the wait of #{at} {rd!r}"

@@ -43,6 +43,25 @@ def test_staircase_triggers_rescales_in_every_wave(chunk_rows):
     assert own_only >= 5 and partner_only >= 5, (own_only, partner_only)
 
 
+@pytest.mark.parametrize("B,chunk_rows", [(24, 1024), (7, 320)])
+@pytest.mark.parametrize("region", [3000, 3072])
+def test_staircase_triggers_rescales_in_the_checked_sequences(B, chunk_rows, region):
+    """The sequences that tests/test_gpu_mfma128.py compares with the oracle: with the chunks of its
+    packed and its 3072-row paged regions, each still moves the maximum of every wave several times."""
+    kv, qa, qr = staircase_case(B, S, "bf16", 5, "cpu")
+    cos, sin = build_rope_tables(S, 64)
+    cos, sin = to_np(cos), to_np(sin)
+    picks = (0, B // 2, B - 1)
+    per_wave = {b: np.zeros(4, int) for b in picks}
+    for b, lo, hi in segments([S] * B, chunk_rows, region):
+        if b not in picks:
+            continue
+        r = lazy_rescale_tiles(scores_log2(to_np(kv[b])[lo:hi], to_np(qa[b]), to_np(qr[b]), cos[lo:hi], sin[lo:hi]))
+        per_wave[b] += [len(set().union(*[set(r[h]) for h in range(32 * w, 32 * w + 32)])) for w in range(4)]
+    for b in picks:
+        assert (per_wave[b] >= 3).all(), (b, per_wave[b])
+
+
 def test_no_rescale_with_gaussian_scores():
     """The contrast: N(0,1) caches and queries (the other GPU tests' inputs)
     never move the running maximum by more than 8 after the first tile."""
