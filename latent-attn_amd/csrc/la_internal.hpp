@@ -322,9 +322,11 @@ __device__ inline int32_t* filled_notes(const DecodeProblem& p) {
 // Partial slot of the piece of chunk c inside sequence s.
 __device__ inline int64_t slot_of(const DecodeProblem& p, int64_t c, int s) { return c + (p.chunk_len < 0 ? 0 : s); }
 // A walk over the segments of one chunk (pieces of it inside one sequence).
-// kFilled: chunk_len may be < 0 (a kernel without it keeps that code, and the
-// registers it holds for later segments, out of its way to the first copy).
-template <bool kFilled>
+// kFilled: 0, chunks of the regions only (such a kernel keeps the other code,
+// and the registers it holds for later segments, out of its way to the first
+// copy); 1, chunk_len may be < 0; 2, it is (one segment: with the code of the
+// others beside it the 128-head kernel's body spilled two registers).
+template <int kFilled>
 struct ChunkWalk {
   int64_t lo, hi;  // what is left of the chunk, in the plan's row space
   int s;           // sequence of the current segment
@@ -332,9 +334,9 @@ struct ChunkWalk {
   int64_t s_lo;    // and in the plan's row space
   int64_t seg_hi;  // end of the current segment there
 };
-template <bool kFilled>
+template <int kFilled>
 __device__ inline bool walk_begin(const DecodeProblem& p, int chunk, int group, ChunkWalk<kFilled>& w) {
-  if (kFilled && p.chunk_len < 0) {
+  if (kFilled == 2 || (kFilled && p.chunk_len < 0)) {
     const FilledPiece f = filled_piece(p, chunk);
     // the last two: malformed offsets, whose sums wrap
     if (f.s >= p.num_seqs || chunk < f.first || (int64_t)(chunk - f.first) * f.len >= f.rows) return false;
@@ -358,10 +360,10 @@ __device__ inline bool walk_begin(const DecodeProblem& p, int chunk, int group, 
   return true;
 }
 // The next segment [lo, seg_hi) of sequence s; after it the caller sets lo = seg_hi and ++s.
-template <bool kFilled>
+template <int kFilled>
 __device__ inline bool walk_next(const DecodeProblem& p, ChunkWalk<kFilled>& w) {
   while (w.lo < w.hi) {
-    if (kFilled && p.chunk_len < 0) return true;  // the one segment, set by walk_begin
+    if (kFilled == 2 || (kFilled && p.chunk_len < 0)) return true;  // the one segment, set by walk_begin
     w.s_lo = w.row0 = seq_begin(p, w.s);
     w.lo = max(w.lo, w.s_lo);  // past the unfilled rows of the previous region
     if (w.lo >= w.hi) return false;

@@ -947,7 +947,7 @@ static_assert(fp8_half_order_ok(), "fp8 expansion halves overlap");
 // kFp8: FP8 E4M3 cache rows (KT = bf16: the tiles are expanded to bf16 in
 // LDS and the MFMAs run on bf16).
 // kFilled: chunks over filled rows (ChunkWalk).
-template <typename KT, bool kPaged, bool kFp8, bool kFilled>
+template <typename KT, bool kPaged, bool kFp8, int kFilled>
 __device__ __forceinline__ void decode_mfma_body(const DecodeProblem& p, int groups) {
   static_assert(!kFp8 || std::is_same<KT, __hip_bfloat16>::value, "fp8 tiles expand to bf16");
   constexpr int kDma = dma_per_wave(kFp8);
@@ -1551,7 +1551,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeProblem& p, int gro
     const int le = lane_id();  // fresh: the prologue's lane index would come back from a spill slot
     const int g2 = le >> 5;
     const float l_tot = sum_halves(l_run);
-    const int64_t slot = kFilled ? slot_of(p, chunk, s) : (int64_t)chunk + s;
+    const int64_t slot = kFilled == 2 ? (int64_t)chunk : kFilled ? slot_of(p, chunk, s) : (int64_t)chunk + s;
     const int64_t hqg = slot * p.Hq + group * kHG;  // slot row of head 0 of the group
     if (le < 32 && 32 * wave + le < hg_heads) {
       p.part_lse[hqg + 32 * wave + le] = m_run + log2f(l_tot);
@@ -1662,6 +1662,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeProblem& p, int gro
     asm volatile("" : "+v"(xb[8]), "+v"(xb[9]), "+v"(xb[10]), "+v"(xb[11]), "+v"(xb[12]), "+v"(xb[13]), "+v"(xb[14]), "+v"(xb[15]));
     store16(par, xb);
     LA_STAMP(9);
+    if constexpr (kFilled == 2) break;  // a piece is one segment
     w.lo = w.seg_hi;
     ++w.s;
   }
@@ -1680,7 +1681,7 @@ __global__ __launch_bounds__(kThreads) void decode_mfma_kernel(DecodeProblem p, 
 // Contiguous capacity caches: the same with chunks over their filled rows.
 template <typename KT, bool kFp8>
 __global__ __launch_bounds__(kThreads) void decode_mfma_filled_kernel(DecodeProblem p, int groups) {
-  decode_mfma_body<KT, false, kFp8, true>(p, groups);
+  decode_mfma_body<KT, false, kFp8, 2>(p, groups);
 }
 
 // Copies-only variant of the attention kernel, for measuring the streaming

@@ -137,3 +137,13 @@ def test_no_register_touched_before_its_wait_on_any_path(decode_asm):
         bad = pending_uses_cfg(lines, counters=("lgkm", "vm"))
         assert not bad, f"{name}: " + "; ".join(f"#{n} {ins!r} before the wait of #{at} {rd!r}"
                                                for n, ins, at, rd in bad[:5])
+
+
+def test_no_attention_kernel_spills(decode_asm):
+    """The kernels hold 256 + 256 registers; one that spills adds scratch traffic to counted waits."""
+    import re
+
+    sizes = dict(re.findall(r"\.amdhsa_kernel (\S+)\n(?:.*\n)*?\s*\.amdhsa_private_segment_fixed_size (\d+)", decode_asm))
+    names = [n for n in sizes if any(n.startswith(k) for k in KERNELS)]
+    assert len(names) == sum(KERNELS.values())
+    assert {n: sizes[n] for n in names if int(sizes[n])} == {}
