@@ -766,10 +766,13 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_half_kernel(Decod
 // column 16 jj + 4 (lane / 16) + e of the half, so both operands come in 16-B
 // loads. Bound by W_UV (33.5 MB at 128 heads) and the partial rows.
 // 4 tokens, 128 heads, 32 slots: 11.8 us; combine_project_kernel, which reduces
-// every output over a wave, 141.
+// every output over a wave, 141. Both halves in one workgroup load a half's
+// weights behind its merge: held through it beside the slot rows and the sums
+// of the other half they spilled 23 registers (32 rows of 100, 128 heads: merge
+// 23.7 us, now 19.8; 64 rows 43.1 and 35.4).
 template <bool F16, bool kHalf>
 __global__ __launch_bounds__(kMPWaves * 64) void merge_project_f32_kernel(DecodeProblem p) {
-  constexpr int kNB = F16 || kHalf ? kMPSlots : kMPSlots / 2;  // fp32 rows, both halves: 8 in flight would spill
+  constexpr int kNB = F16 || kHalf ? kMPSlots : kMPSlots / 2;  // both halves and fp32 rows: 8 do not fit beside the sums
   warm_kernarg_lines(p);
   __shared__ __attribute__((aligned(16))) float orow[kMPRows * kMPHSum];  // merged half rows
   __shared__ __attribute__((aligned(16))) float gp[kMPWaves * kMPHSum];   // slot-group sums
@@ -789,8 +792,11 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_f32_kernel(Decode
   const int c_first = kHalf ? (k & 1) : 0, c_end = kHalf ? c_first + 1 : 2;
   for (int c = c_first; c < c_end; ++c) {
     f32x4 bw[16];
+    auto load_w = [&] {
 #pragma unroll
-    for (int jj = 0; jj < 16; ++jj) bw[jj] = *reinterpret_cast<const f32x4*>(wrow + 256 * c + 16 * jj);
+      for (int jj = 0; jj < 16; ++jj) bw[jj] = *reinterpret_cast<const f32x4*>(wrow + 256 * c + 16 * jj);
+    };
+    if (kHalf) load_w();
     if (c > c_first) __syncthreads();  // every wave is done with the first half's rows
     f32x4 o[2][2];
     if (rows >= kMPWaves) {
@@ -814,6 +820,7 @@ __global__ __launch_bounds__(kMPWaves * 64) void merge_project_f32_kernel(Decode
         *reinterpret_cast<f32x4*>(&orow[rr * kMPHSum + 4 * c4]) = v;
       }
     }
+    if (!kHalf) load_w();
     __syncthreads();
     // A[m = lane % 16][latent column] from LDS, B[latent column][n = lane % 16] = W_UV
 #pragma unroll

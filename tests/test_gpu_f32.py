@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from conftest import assert_close
-from mla_cases import cfg_with_heads, make_queries, make_weights, rope, staircase_case, to_np
+from mla_cases import TORCH_DTYPE, cfg_with_heads, make_queries, make_weights, rope, staircase_case, to_np
 from oracle import mla_oracle as mo
 from test_gpu_plan import F32, VALU, plan
 
@@ -174,3 +174,25 @@ def test_workspace_that_is_only_float_aligned(cuda, heads, shift):
     ref = mo.decode_sequences(to_np(kv), [0, S, 2 * S], mo.absorb_q(to_np(q_nope), to_np(W_UK), d), to_np(q_rope),
                               to_np(W_UV), to_np(cos), to_np(sin), d)
     assert_close(out.cpu().numpy(), ref, "f32", f"f32 H={heads}, workspace + {shift} B")
+
+
+@pytest.mark.parametrize("cache", ["f32", "bf16"])
+@pytest.mark.parametrize("B,S", [(17, 70), (33, 40), (20, 300)])
+def test_full_merge(cuda, cache, B, S):
+    """float32 weights and enough query rows for the merge of both latent halves in one workgroup
+    (two blocks of 16 rows or three, the last with one), over fp32 and fp16 partial rows."""
+    from latent_attn import functional as F
+
+    cfg = cfg_with_heads(128)
+    if torch.cuda.get_device_properties(cuda).multi_processor_count == 256:
+        assert plan(cache, 128, B, S, wdtype="f32", chunk_rows=64).merge == capi.LA_PLAN_MERGE_MFMA_F32
+    W_UK, W_UV = make_weights(cfg, "f32", 21, cuda)
+    q_nope, q_rope = make_queries((B,), cfg, 22, cuda)
+    cos, sin = rope(S, cfg, cuda)
+    kv = torch.randn(B, S, 576, generator=torch.Generator().manual_seed(23)).to(TORCH_DTYPE[cache]).to(cuda)
+    out = F.mla_decode(kv, q_nope, q_rope, W_UK, W_UV, cos, sin, cfg, chunk_rows=64).cpu().numpy()
+    d = _dims(cfg)
+    ref = mo.decode_sequences(to_np(kv).reshape(B * S, 576), [b * S for b in range(B + 1)],
+                              mo.absorb_q(to_np(q_nope), to_np(W_UK), d), to_np(q_rope), to_np(W_UV), to_np(cos),
+                              to_np(sin), d)
+    assert_close(out, ref, cache, f"full fp32 merge, {cache} cache, {B} rows")
