@@ -140,9 +140,10 @@ typedef struct la_decode_args {
    * them): sequence s is the first seq_lens[s] rows of its region above
    * (clamped into it; rows past it are unfilled capacity and are not read).
    * NULL: each sequence is its whole region. The MFMA kernels cut the
-   * filled rows (unless chunk_rows is given, or there are fewer than four
-   * chunks per sequence); otherwise the split plan covers the regions, so
-   * capacity far beyond the lengths costs idle blocks. */
+   * filled rows (unless chunk_rows is given, there are fewer than four chunks
+   * per sequence, or the pieces would be the regions' chunks: la_plan_info's
+   * filled_rows); otherwise the split plan covers the regions, so capacity far
+   * beyond the lengths costs idle blocks. */
   const int32_t* seq_lens;
   /* optional paged cache (block tables): kv_cache is then a pool of
    * total_rows rows in blocks of block_size rows (total_rows a multiple of

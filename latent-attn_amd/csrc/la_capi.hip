@@ -1,7 +1,11 @@
 // extern "C" entry points of liblatent_attn_hip.so (declared in
 // include/latent_attn.h): argument checking, split-KV planning, workspace
-// carving and kernel dispatch. Host code only; the kernels live in
-// la_generic.hip and la_mfma.hip.
+// carving and kernel dispatch. Host code only; the kernels live in the other
+// files: attention in la_mfma.hip (128 heads a workgroup), la_mfma16.hip (16),
+// la_f32.hip (float32) and la_generic.hip (any shape), absorption and merge +
+// projection for 16-bit weights and the merge for float32 ones in la_proj.hip,
+// the other absorption in la_f32.hip and la_generic.hip, la_append.hip,
+// la_naive.hip.
 #include "la_internal.hpp"
 
 #include <algorithm>
@@ -71,7 +75,8 @@ struct Plan {
 // Fills the problem (without workspace pointers) and the plan. The args'
 // chunk_rows / kernel_variant fields are tuning overrides (0 = automatic).
 // coarse: the chunks of one 128-head (or VALU) workgroup per target block, also
-// for the kernels with 16 heads per workgroup: fewer partial slots, for a caller whose scratch does not hold the others.
+// for the kernels with 16 heads per workgroup: fewer partial slots, for a caller
+// whose scratch does not hold the others.
 int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse = false) {
   if (!a || !valid_cfg(&a->cfg)) return LA_ERROR_INVALID_VALUE;
   const int chunk_rows = a->chunk_rows;
@@ -291,7 +296,8 @@ int prepare(const la_decode_args* a, DecodeProblem* p, Plan* plan, bool coarse =
 // merge, so it is split over the two latent halves, which add into the
 // output (zeroed first by the kernel that writes the attention kernel's
 // 16-bit queries: the absorb kernel, or prep_q when the queries come
-// absorbed and there is at least one chunk).
+// absorbed and there is at least one chunk; where the attention kernel takes
+// the fp32 queries itself, by that one).
 bool merge_halves(const DecodeProblem& p, const Plan& plan) {
   const bool zeroed = plan.f32 ? plan.num_chunks > 0  // by decode_f32_kernel itself
                                : plan.mfma && (plan.absorb_prep || plan.num_chunks > 0);
@@ -350,14 +356,14 @@ int run(const la_decode_args* a, hipStream_t stream, hipEvent_t ev_b = nullptr, 
                              c.qk_nope_head_dim, c.kv_lora_rank, a->queries_per_seq, stream, zero_out, zero_n);
     } else {
       float* qa = reinterpret_cast<float*>(ws + plan.q_abs_off);
-      e = plan.absorb_f32 ? launch_absorb_f32(a->q_nope, a->W_UK, qa, (int)tokens, c.num_heads, c.qk_nope_head_dim,
-                                              c.kv_lora_rank, stream)
-          : plan.absorb_mfma
-              ? launch_absorb_mfma(a->q_nope, a->W_UK, a->w_uk_dtype, qa, 0, nullptr, 1.f, 0,
-                                                (int)tokens, c.num_heads, c.qk_nope_head_dim, c.kv_lora_rank, 1,
-                                                stream)
-                           : launch_absorb(a->q_nope, a->W_UK, a->w_uk_dtype, qa, (int)tokens, c.num_heads,
-                                           c.qk_nope_head_dim, c.kv_lora_rank, stream);
+      if (plan.absorb_f32)
+        e = launch_absorb_f32(a->q_nope, a->W_UK, qa, (int)tokens, c.num_heads, c.qk_nope_head_dim, c.kv_lora_rank, stream);
+      else if (plan.absorb_mfma)
+        e = launch_absorb_mfma(a->q_nope, a->W_UK, a->w_uk_dtype, qa, 0, nullptr, 1.f, 0, (int)tokens, c.num_heads,
+                               c.qk_nope_head_dim, c.kv_lora_rank, 1, stream);
+      else
+        e = launch_absorb(a->q_nope, a->W_UK, a->w_uk_dtype, qa, (int)tokens, c.num_heads, c.qk_nope_head_dim,
+                          c.kv_lora_rank, stream);
       p.q_abs = qa;
     }
     if (e != hipSuccess) return finish(e);
@@ -385,16 +391,16 @@ int run(const la_decode_args* a, hipStream_t stream, hipEvent_t ev_b = nullptr, 
     } else {
       if (ev_b) e = hipEventRecord(ev_b, stream);
       for (int r = 0; r < reps && e == hipSuccess; ++r)
-        e = plan.mfma ? launch_mfma(nullptr, nullptr)
+        e = plan.mfma  ? launch_mfma(nullptr, nullptr)
             : plan.f32 ? launch_decode_f32(p, stream, zero_out, zero_n)
                        : launch_decode_generic(p, stream);
       if (e == hipSuccess && ev_e) e = hipEventRecord(ev_e, stream);
     }
     if (e != hipSuccess) return finish(e);
   }
-  return finish(plan.proj_f32 ? launch_combine_project_f32(p, stream, merge_halves)
-                : plan.proj_mfma ? launch_combine_project_mfma(p, stream, merge_halves, cu_count())
-                                : launch_combine_project(p, stream));
+  if (plan.proj_f32) return finish(launch_combine_project_f32(p, stream, merge_halves));
+  if (plan.proj_mfma) return finish(launch_combine_project_mfma(p, stream, merge_halves, cu_count()));
+  return finish(launch_combine_project(p, stream));
 }
 
 la_decode_args shared_cache_args(const void* kv_cache, int kv_dtype, int seq_len, int batch, const float* q_absorbed,

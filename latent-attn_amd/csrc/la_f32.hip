@@ -8,10 +8,13 @@
 // read every row 128 times through the L2 and reduce every score over a wave:
 // 4 x 1000 rows and 128 heads took 377 us. Here a workgroup of 4 waves takes 16
 // heads and walks tiles of 32 positions staged in LDS; two workgroups share a
-// CU (74 KB each), one's loads under the other's matrix work.
+// CU (76 KB each), one's loads under the other's matrix work.
 // 4 x 1000 rows and 128 heads take 32.6 us (17.4K of 53K cycles in the matrix
 // cores; the rest is the latency of loads, barriers and softmax, which two
-// workgroups only partly hide), 1 x 8192 37 us.
+// workgroups only partly hide), 1 x 8192 37 us. Fewer heads than 16 multiply the
+// 16-head tile all the same and gain as much (a whole step of one head, here and
+// on decode_generic_kernel: 1 x 64 rows 26 / 152 us, 1 x 8192 30 / 415, 64 x 10
+// 64 / 186).
 //
 // An MFMA step multiplies 4 k's, lane group g = lane / 16 holding one of them;
 // which k's a step takes is free as long as both operands agree, so every
@@ -56,11 +59,7 @@ __device__ inline f32x4 lds_ld(const lchar* L, int off) {
 __device__ inline void lds_st(lchar* L, int off, f32x4 v) {
   *reinterpret_cast<__attribute__((address_space(3))) f32x4*>(L + off) = v;
 }
-__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ inline f32x4 mma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-// 16 wait states between the last MFMA writing d and its first VALU reader
-// (the compiler adds none where a branch lies between the two).
-__device__ inline void settle(f32x4& d) { asm volatile("s_nop 15" : "+v"(d)); }
 
 template <bool kPaged, bool kFilled>
 __global__ __launch_bounds__(kThreads, 2) void decode_f32_kernel(DecodeProblem p, int groups, float* zero_out,
@@ -120,8 +119,8 @@ __global__ __launch_bounds__(kThreads, 2) void decode_f32_kernel(DecodeProblem p
       const int left = last - tb;
       const char* base;
       if constexpr (kPaged) {
-        const uint32_t pos = pos0 + (uint32_t)tb, q32 = pos >> 5;
-        const uint32_t blk = (__umulhi(q32, p.tpb_magic) + q32) >> p.tpb_shift;
+        const uint32_t pos = pos0 + (uint32_t)tb, tile = pos >> 5;
+        const uint32_t blk = (__umulhi(tile, p.tpb_magic) + tile) >> p.tpb_shift;
         const int e = min(max(p.block_table[(int64_t)s * p.blocks_per_seq + blk], 0), p.pool_last);
         const uint32_t row = (uint32_t)e * (uint32_t)p.block_size + (pos - blk * (uint32_t)p.block_size);
         base = reinterpret_cast<const char*>(p.kv) + (uint64_t)row * kRowB;

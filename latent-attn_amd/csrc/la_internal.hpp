@@ -237,8 +237,8 @@ __device__ inline int find_seq_mfma(const DecodeProblem& p, int64_t r) {
 // attention kernel sums them itself (wave-uniform code, all lanes active), and
 // its workgroups leave what the merge needs in free slots
 // (filled_notes): summed again there, behind its weight loads, it cost 1.5 us.
-// The lane index is made in an asm statement at each use: held in a register
-// for later segments it would spill beside the 128-head kernel's operands.
+// The lane index is made in a volatile asm statement at each use, so that what
+// derives from it is not held across loops, beside the operands in registers.
 __device__ inline int wave_lane() {
   int l;
   asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
@@ -453,6 +453,23 @@ __device__ inline float load_any(const void* base, int dtype, int64_t i) {
   if (dtype == LA_DTYPE_F16) return __half2float(reinterpret_cast<const __half*>(base)[i]);
   if (dtype == LA_DTYPE_FP8_E4M3) return fp8_to_f32(reinterpret_cast<const uint8_t*>(base)[i]);
   return reinterpret_cast<const float*>(base)[i];
+}
+
+// LDS-visibility barrier that leaves outstanding HBM->LDS copies in flight.
+// The "memory" clobber keeps the compiler from moving LDS accesses across it.
+__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// 16 wait states between the last MFMA writing d and its first VALU reader (the
+// compiler adds none where a branch lies between the two: row maxima were taken
+// of unfinished scores).
+template <typename V>
+__device__ inline void settle(V& d) { asm volatile("s_nop 15" : "+v"(d)); }
+
+__device__ inline float f_of(unsigned u) { return __builtin_bit_cast(float, u); }
+__device__ inline unsigned u_of(float f) { return __builtin_bit_cast(unsigned, f); }
+// x[l] + x[l ^ 32]
+__device__ inline float sum_halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(u_of(x), u_of(x), false, false);
+  return f_of(r[0]) + f_of(r[1]);
 }
 
 __device__ inline float wave_sum(float v) {

@@ -393,10 +393,6 @@ constexpr int qb_vm_n() {
   return (30 - KK) + c + (Paged ? 1 : 0);
 }
 
-// LDS-visibility barrier that leaves outstanding HBM->LDS copies in flight.
-// The "memory" clobber keeps the compiler from moving LDS accesses across it.
-__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // The lane index, computed by a volatile asm (v_mbcnt) at each use: nothing
 // derived from it can be hoisted out of the enclosing loop, so per-lane
 // addresses are recomputed per tile (a few VALU ops) instead of being kept
@@ -412,13 +408,6 @@ __device__ inline int lane_id() {
 // returns (x[l % 32], x[l % 32 + 32]) in every lane l, permlane16_swap(x, x)
 // the same for 16-lane halves of each 32-lane half; DPP 0xB1 / 0x4E / 0x141
 // / 0x140 read lane l^1 / l^2 / the mirror inside 8 / inside 16 lanes.
-__device__ inline float f_of(unsigned u) { return __builtin_bit_cast(float, u); }
-__device__ inline unsigned u_of(float f) { return __builtin_bit_cast(unsigned, f); }
-// x[l] + x[l ^ 32]
-__device__ inline float sum_halves(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(u_of(x), u_of(x), false, false);
-  return f_of(r[0]) + f_of(r[1]);
-}
 // max of x over lanes l^32
 __device__ inline float max_halves(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(u_of(x), u_of(x), false, false);

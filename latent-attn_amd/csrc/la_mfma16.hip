@@ -127,22 +127,7 @@ __device__ inline void lds_st(lchar* L, int off, T v) {
 __device__ inline i16x4 lds_tr(const lchar* L, int off) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(lds_void*)(L + off));
 }
-__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// The lane index from a volatile asm: what derives from it is not hoisted out of the loops.
-__device__ inline int fresh_lane() {
-  int l;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-  return l;
-}
-
-// 16 wait states between the last MFMA writing d and its first VALU reader (the
-// compiler adds none where a branch lies between the two: row maxima were
-// taken of unfinished scores).
-__device__ inline void settle(f32x4& d) { asm volatile("s_nop 15" : "+v"(d)); }
-
-__device__ inline float f_of(unsigned u) { return __builtin_bit_cast(float, u); }
-__device__ inline unsigned u_of(float f) { return __builtin_bit_cast(unsigned, f); }
 // max / sum of x over the four lanes l%16 + 16 g
 __device__ inline float max_groups(float x) {
   auto r = __builtin_amdgcn_permlane32_swap(u_of(x), u_of(x), false, false);
@@ -212,7 +197,7 @@ __global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem
     const bool q32 = kW == 8 && !p.q_prep;
     f32x4 qf[kW == 8 ? 6 : 1];
     if (!q32) {
-      const int ql = fresh_lane();
+      const int ql = wave_lane();
       const int64_t qrow = (int64_t)s * qprep_rows_per_seq(p.Hq) + head0 + (ql & 15);
       const vec* qs =
           reinterpret_cast<const vec*>(reinterpret_cast<const E*>(p.q_prep) + qprep_index(qrow, 8 * (ql >> 4)));
@@ -240,14 +225,14 @@ __global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem
     for (int t = 0; t < ntiles; ++t) {
       // the tile's LDS addresses are made where they are used, from a fresh
       // lane index (held across the loop they would not fit beside Q and O)
-      const int ln = fresh_lane();
+      const int ln = wave_lane();
       // ---- stage the wave's 16 rows (rows past the segment re-read its last) ----
       const int pb = min(kT * t + 16 * wave, last);  // first row; the 16 lie in one block of a paged cache
       const int left = last - pb;
       const char* base;
       if constexpr (kPaged) {
-        const uint32_t pos = pos0 + (uint32_t)pb, q32 = pos >> 5;
-        const uint32_t blk = (__umulhi(q32, p.tpb_magic) + q32) >> p.tpb_shift;
+        const uint32_t pos = pos0 + (uint32_t)pb, tile = pos >> 5;
+        const uint32_t blk = (__umulhi(tile, p.tpb_magic) + tile) >> p.tpb_shift;
         const int e = min(max(p.block_table[(int64_t)s * p.blocks_per_seq + blk], 0), p.pool_last);
         const uint32_t row = (uint32_t)e * (uint32_t)p.block_size + (pos - blk * (uint32_t)p.block_size);
         base = reinterpret_cast<const char*>(p.kv) + (uint64_t)row * kRowB;
@@ -429,7 +414,7 @@ __global__ __launch_bounds__(64 * kW, 2) void decode_mfma16_kernel(DecodeProblem
     // ---- segment end: the partial slot's rows, as decode_mfma_kernel writes them ----
     // fp16 N * 2^-e per half row, 2^(e-1) <= max |N| < 2^e; m and m + log2(l)
     lds_barrier();  // every wave is done with the tile
-    const int lane = fresh_lane();
+    const int lane = wave_lane();
     const int n16 = lane & 15, g = lane >> 4;
     const int64_t hq0 = (kFilled ? slot_of(p, chunk, s) : (int64_t)chunk + s) * p.Hq + head0;
     float rmax = 0.f;

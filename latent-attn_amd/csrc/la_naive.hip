@@ -211,14 +211,6 @@ constexpr int kMmThreads = 512;
 // a stage: position rows, then weight rows, 64 B each; chunk j of row r at j ^ sw(r)
 constexpr int kStageBytes = (kPos + kHd) * kBk * 2;
 __device__ inline int sw(int r) { return (r >> 2) & 3; }
-__device__ inline float f_of(unsigned u) { return __builtin_bit_cast(float, u); }
-// x[l] + x[l ^ 32]
-__device__ inline float sum_halves(float x) {
-  const unsigned u = __builtin_bit_cast(unsigned, x);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return f_of(r[0]) + f_of(r[1]);
-}
-
 // acc[i][j] of wave (wa, wb) = rows 64 wa + 32 i of the M operand times rows
 // 64 wb + 32 j of the N operand, over K columns; the M operand is the weights
 // (kWeightsM) or the positions. Every stage is three 1-KB HBM->LDS copies per
