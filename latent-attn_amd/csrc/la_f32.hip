@@ -9,8 +9,8 @@
 // 4 x 1000 rows and 128 heads took 377 us. Here a workgroup of 4 waves takes 16
 // heads and walks tiles of 32 positions staged in LDS; two workgroups share a
 // CU (76 KB each), one's loads under the other's matrix work.
-// 4 x 1000 rows and 128 heads take 32.6 us (17.4K of 53K cycles in the matrix
-// cores; the rest is the latency of loads, barriers and softmax, which two
+// 4 x 1000 rows and 128 heads take 33 us (matrix cores 17.4K of 58.6K busy
+// cycles; the rest is the latency of loads, barriers and softmax, which two
 // workgroups only partly hide), 1 x 8192 37 us. Fewer heads than 16 multiply the
 // 16-head tile all the same and gain as much (a whole step of one head, here and
 // on decode_generic_kernel: 1 x 64 rows 26 / 152 us, 1 x 8192 30 / 415, 64 x 10
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(kThreads, 2) void decode_f32_kernel(DecodeProblem p
 // (head, 64 latent columns, 16 tokens): step (jj, e) takes i = 16 jj + 4 g + e,
 // A = W's row i, 4 consecutive columns per lane (one per MFMA), B = q. W
 // streams through registers once per 16 tokens (33.5 MB at 128 heads), eight
-// 16-row groups of loads in flight per wave: 7.9 us for 4 tokens, where
+// 16-row groups of loads in flight per wave: 9.6 us for 4 tokens, where
 // absorb_kernel (one column per thread, serial over i) took 52.8.
 // kNJ = dn / 16 when known at compile time (8 for dn = 128), 0 for any multiple
 // of 16.

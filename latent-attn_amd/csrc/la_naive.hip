@@ -14,7 +14,8 @@
 // workgroup decompresses 256 positions of one head and either dots them with
 // the head's query (naive_k_kernel) or weights and sums them
 // (naive_v_kernel). At S = 8192 and 128 heads the two products are 275 GFLOP:
-// about 150 us each (0.9 PFLOP/s), 329 us a call with the rest.
+// 157 to 172 us each (0.8 to 0.87 PFLOP/s; matrix cores busy half of it), 329 us
+// a call with the rest.
 // Other types and shapes take the plain kernels: a 64x64-tiled VALU GEMM into
 // fp32 K_nope and V, one thread per (head, position) for the scores, one
 // workgroup per head for the softmax and the weighted sum (10.2 ms there).
