@@ -220,13 +220,13 @@ bool append_vec(const AppendProblem& p) {
 hipError_t launch_append(const AppendProblem& p, hipStream_t stream) {
   if (p.num_seqs == 0) return hipSuccess;
   // One element per thread while that is one round (a decode step's token), or,
-  // into an FP8 cache, up to two and a half: the software conversions of eight
-  // in one thread are a longer chain (64 sequences, FP8 from fp32 with a fill
-  // launch, one against eight elements per thread: 2 tokens of 576 4.70 / 5.04 us,
-  // 4 tokens 5.36 / 5.28, 5 tokens 5.85 / 5.25; from FP8 4 tokens 5.62 / 5.80; bf16
-  // 2 tokens 4.83 / 4.42).
+  // into an FP8 cache, one and a half: the software conversions of eight in one
+  // thread are a longer chain (64 sequences, FP8 from fp32 with a fill launch, one
+  // against eight elements per thread: 2 tokens of 576 4.70 / 5.04 us, 3 tokens
+  // 5.05 / 5.06, 4 tokens with rotated queries 6.40 / 5.98, 5 tokens 5.85 / 5.25;
+  // bf16 2 tokens 4.83 / 4.42).
   const int64_t elems = (int64_t)p.tokens * (p.dc + p.dR);
-  const bool vec = 2 * elems > (p.kv_dtype == LA_DTYPE_FP8_E4M3 ? 5 : 2) * kAppendThreads && append_vec(p);
+  const bool vec = 2 * elems > (p.kv_dtype == LA_DTYPE_FP8_E4M3 ? 3 : 2) * kAppendThreads && append_vec(p);
   const int half = p.dR / 2;
   const int64_t rows_n = elems / (vec ? 8 : 1);
   const int64_t quer_n = p.q_rope ? (int64_t)p.qps * p.nh * (half % 4 == 0 ? half / 4 : half) : 0;
