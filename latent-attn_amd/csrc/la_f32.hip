@@ -316,13 +316,9 @@ __global__ __launch_bounds__(256) void absorb_f32_kernel(const float* __restrict
 
 template <bool kPaged, bool kFilled>
 hipError_t launch_f32_t(const DecodeProblem& p, hipStream_t stream, float* zero_out, int64_t zero_n) {
-  static bool attr_set = false;  // per instance; setting it twice is harmless
-  if (!attr_set) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_f32_kernel<kPaged, kFilled>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
+  static OncePerDevice once;
+  const hipError_t e = allow_lds(once, reinterpret_cast<const void*>(&decode_f32_kernel<kPaged, kFilled>), kLdsBytes);
+  if (e != hipSuccess) return e;
   const int groups = (p.Hq + 15) / 16;
   hipLaunchKernelGGL((decode_f32_kernel<kPaged, kFilled>), dim3((unsigned)mfma_grid_blocks(p.num_chunks, groups)), dim3(kThreads),
                      kLdsBytes, stream, p, groups, zero_out, zero_n);

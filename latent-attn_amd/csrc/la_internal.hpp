@@ -8,6 +8,7 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "la_once.hpp"
 #include "latent_attn.h"
 
 namespace la {
@@ -547,6 +548,14 @@ hipError_t launch_append(const AppendProblem& p, hipStream_t stream);
 // VALU split-KV decode: any dtype, kv_lora_rank <= 1024, qk_rope_head_dim <= 256.
 hipError_t launch_decode_generic(const DecodeProblem& p, hipStream_t stream);
 bool generic_supported(const DecodeProblem& p);
+
+// Raises a kernel's dynamic LDS limit on the current device; each kernel has an OncePerDevice of its own.
+inline hipError_t allow_lds(OncePerDevice& once, const void* fn, int bytes) {
+  int dev = 0;
+  const hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  return once.run(dev, [&] { return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes); });
+}
 
 // Whether the current device runs the MFMA kernels.
 bool device_is_gfx950();

@@ -1785,18 +1785,20 @@ __global__ __launch_bounds__(256) void prep_q_kernel(const float* __restrict__ q
   *reinterpret_cast<vec*>(out + qprep_index(qrow, 8 * j)) = v;
 }
 
-hipError_t launch_k(void (*k)(DecodeProblem, int), bool* attr_set, const DecodeProblem& p, hipStream_t stream,
+hipError_t launch_k(void (*k)(DecodeProblem, int), OncePerDevice& once, const DecodeProblem& p, hipStream_t stream,
                     hipEvent_t ev_begin, hipEvent_t ev_end) {
-  if (!*attr_set) {  // per kernel; setting it twice is harmless
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  e = once.run(dev, [&] {
     const void* fn = reinterpret_cast<const void*>(k);
     hipFuncAttributes fa;
-    hipError_t e = hipFuncGetAttributes(&fa, fn);
-    if (e != hipSuccess) return e;
+    const hipError_t f = hipFuncGetAttributes(&fa, fn);
+    if (f != hipSuccess) return f;
     if (fa.sharedSizeBytes != 0) return hipErrorInvalidKernelFile;  // LDS offsets would not be addresses
-    e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-    if (e != hipSuccess) return e;
-    *attr_set = true;
-  }
+    return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+  });
+  if (e != hipSuccess) return e;
   const int groups = (p.Hq + kHG - 1) / kHG;
   const dim3 blocks((unsigned)mfma_grid_blocks(p.num_chunks, groups));
   if (ev_begin || ev_end)  // the events time this kernel's execution alone (no dispatch gap)
@@ -1808,10 +1810,10 @@ hipError_t launch_k(void (*k)(DecodeProblem, int), bool* attr_set, const DecodeP
 
 template <typename KT, bool kFp8>
 hipError_t launch_t(const DecodeProblem& p, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
-  static bool set[3] = {false, false, false};
-  if (p.block_table) return launch_k(decode_mfma_kernel<KT, true, kFp8>, &set[0], p, stream, ev_begin, ev_end);
-  if (p.chunk_len < 0) return launch_k(decode_mfma_filled_kernel<KT, kFp8>, &set[1], p, stream, ev_begin, ev_end);
-  return launch_k(decode_mfma_kernel<KT, false, kFp8>, &set[2], p, stream, ev_begin, ev_end);
+  static OncePerDevice once[3];
+  if (p.block_table) return launch_k(decode_mfma_kernel<KT, true, kFp8>, once[0], p, stream, ev_begin, ev_end);
+  if (p.chunk_len < 0) return launch_k(decode_mfma_filled_kernel<KT, kFp8>, once[1], p, stream, ev_begin, ev_end);
+  return launch_k(decode_mfma_kernel<KT, false, kFp8>, once[2], p, stream, ev_begin, ev_end);
 }
 
 }  // namespace

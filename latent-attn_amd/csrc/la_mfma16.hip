@@ -472,13 +472,9 @@ template <typename KT, int kW, bool kPaged, bool kFp8, bool kFilled>
 hipError_t launch16_t(const DecodeProblem& p, hipStream_t stream, float* zero_out, int zero_n, hipEvent_t ev_begin,
                       hipEvent_t ev_end) {
   constexpr int lds = Lds<kW>::kBytes;
-  static bool attr_set = false;  // per instance; setting it twice is harmless
-  if (!attr_set) {
-    const void* fn = reinterpret_cast<const void*>(&decode_mfma16_kernel<KT, kW, kPaged, kFp8, kFilled>);
-    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
+  static OncePerDevice once;
+  const hipError_t e = allow_lds(once, reinterpret_cast<const void*>(&decode_mfma16_kernel<KT, kW, kPaged, kFp8, kFilled>), lds);
+  if (e != hipSuccess) return e;
   const int groups = p.Hq / 16;
   const dim3 grid((unsigned)mfma_grid_blocks(p.num_chunks, groups));
   if (ev_begin || ev_end)

@@ -465,22 +465,17 @@ bool naive_mm_supported(const NaiveProblem& p) {
 template <typename T>
 hipError_t run_naive_mm(const NaiveProblem& p, hipStream_t stream) {
   constexpr int lds = kStages * kStageBytes;
-  static bool attr_set = false;  // per instance; setting it twice is harmless
-  if (!attr_set) {
-    for (const void* fn : {reinterpret_cast<const void*>(&naive_k_kernel<T>), reinterpret_cast<const void*>(&naive_v_kernel<T>)}) {
-      const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-      if (e != hipSuccess) return e;
-    }
-    attr_set = true;
-  }
+  static OncePerDevice once_k, once_v;
+  hipError_t e = allow_lds(once_k, reinterpret_cast<const void*>(&naive_k_kernel<T>), lds);
+  if (e == hipSuccess) e = allow_lds(once_v, reinterpret_cast<const void*>(&naive_v_kernel<T>), lds);
+  if (e != hipSuccess) return e;
   const int blocks = (p.S + kPos - 1) / kPos;
   const T* kv = reinterpret_cast<const T*>(p.kv);
   const dim3 rgrid((unsigned)((p.S + 63) / 64), (unsigned)((p.nh + kRopeHeads - 1) / kRopeHeads));
   const dim3 grid((unsigned)(8 * ((p.nh + 7) / 8) * blocks));
   hipLaunchKernelGGL(naive_rope_kernel<T>, rgrid, dim3(256), 0, stream, kv, p.S, p.dc, p.nh, p.q_rope, p.rope_cos,
                      p.rope_sin, p.rope_rows, p.scale, p.scores);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL(naive_k_kernel<T>, grid, dim3(kMmThreads), lds, stream, kv, p.S, p.dc, p.dR,
                      reinterpret_cast<const T*>(p.W_UK), p.nh, p.q_nope, p.scale, p.scores);
   if ((e = hipGetLastError()) != hipSuccess) return e;
